@@ -6,15 +6,21 @@
 //   * capability filter: the entry's precision, a gfx950 device, 32-bit offsets and grid limits
 //     (gie_hip_f32_check), split <= the number of (tap, 16-channel) stages;
 //   * workspace: none for split 1; split * |Y| FP32 partials otherwise (reduced by gie_hip_splitk_reduce).
+//   * the 64-filter split-1 entry runs whichever of its tile kernel and the small-convolution kernel (conv_mini.hip) is
+//     expected to be faster: the tile kernel reads each stage one stage ahead and needs hundreds of 64 x 128 tiles,
+//     the other splits the reduction inside a workgroup (one image 3x3 64 -> 64 over 56x56: 6.6 us against 18.3 with
+//     eight split-K slices and their reduce).
 // The FP32 matrix-core rate equals the vector FP32 rate on gfx950 (256 FLOP/clk/CU), so the cost model prices
 // these entries against the FP32 ceiling (uses_tensor_cores = false).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
 #include "gie_hip.h"
 #include "gpu_inference/kernel_registry.h"
+#include "mini_family.h"
 
 namespace gie {
 namespace {
@@ -76,6 +82,26 @@ struct Fns {
     return Split > 1 ? 2.0 * Split * double(prob.p.output_shape().numel()) * 4.0 : 0.0;
   }
   static int occupancy(const ConvProblem&) { return 2; }
+  // The tile kernel: 1.3 us (64 filters) or 2.9 us (128) for each 16-channel stage of a CU's share of the workgroups
+  // (1x1 256 -> 1024, 6272 pixels: 65.9 and 74.1 us), then the split-K reduce at about 4 TB/s of partials.
+  static double tile_us(const ConvProblem& prob, int cus) {
+    const Conv2DParams& p = prob.p;
+    const double stages = double(p.kernel_h) * p.kernel_w * ((p.in_channels + 15) / 16) / Split;
+    const double share = std::max(1.0, double(blocks(prob)) / std::max(cus, 1));
+    return 1.0 + share * stages * (tile_m() == 64 ? 1.3 : 2.9) +
+           (Split > 1 ? 1.0 + (Split + 1) * double(p.output_shape().numel()) * 4.0 / 4e6 : 0.0);
+  }
+  // the small-convolution configuration that runs this problem in the entry's place, or -1
+  static int mini_config(const ConvProblem& prob, int cus) {
+    if (Split != 1 || tile_m() != 64) return -1;
+    double us = 0;
+    const int c = mini_best_config(prob, cus, &us);
+    return c >= 0 && us < tile_us(prob, cus) ? c : -1;
+  }
+  static double busy_us(const ConvProblem& prob, int cus) {
+    const int c = mini_config(prob, cus);
+    return c >= 0 ? mini_busy_us(c, prob, cus) : tile_us(prob, cus);
+  }
   static void launch(const LaunchArgs& la) {
     const ConvProblem& prob = *la.problem;
     const gie_conv_geom g = geom_of(prob);
@@ -83,6 +109,11 @@ struct Fns {
     const auto stage = [&](int k) { return la.only_stage < 0 || la.only_stage == k; };
     // stage 1: the convolution (no repack stage); stage 2: the split-K reduce
     if (stage(1)) {
+      const int mini = mini_config(prob, la.dev->sm_count);
+      if (mini >= 0) {
+        mini_launch(mini, prob, la.x, la.w, la.bias, la.y, la.stream);
+        return;
+      }
       check_kernel_status(gie_hip_conv_f32(Config, dtype_of(P), &g, la.x, la.w, la.bias, la.y, part, Split, la.stream),
                           "FP32 MFMA convolution");
     }
@@ -121,6 +152,7 @@ KernelDesc make_entry() {
   k.num_blocks = &F::blocks;
   k.extra_traffic_bytes = &F::extra_traffic;
   k.blocks_per_cu = &F::occupancy;
+  k.busy_us = &F::busy_us;
   k.launch = &F::launch;
   return k;
 }

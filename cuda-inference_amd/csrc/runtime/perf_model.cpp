@@ -6,6 +6,7 @@
 //   memory  = (compulsory bytes + the kernel's extra traffic) / (HBM bandwidth x family HBM efficiency)
 //   fixed   = launches x dispatch cost + the family's cost of filling and draining a launch
 //   time    = max(compute, memory) + fixed      (reported as launch_us; "launch"-bound when it dominates)
+// A family with a formula of its own (KernelDesc::busy_us: everything but dispatch) takes that as its compute time.
 // * Family efficiencies are not guesses per backend: each is what that kernel family reached on an MI355X in the
 //   library's benchmark protocol (per-call time, inputs resident in HBM), listed in kFamilies with the measurement.
 // * Wave efficiency follows how gfx950 places workgroups: dispatch deals them round-robin to the 8 XCDs, and each
@@ -299,11 +300,12 @@ Estimate estimate_kernel(const ConvProblem& prob, const KernelDesc& k, const Dev
   const double peak_tflops = k.uses_tensor_cores ? c.fp16_tc_tflops : c.fp32_tflops;
   const double rate = peak_tflops * 1e6 * mfma_eff * std::max(e.tile_efficiency, 1e-3) *
                       std::max(e.wave_efficiency, 1e-3);  // FLOP per us
-  e.compute_us = m.flops / rate;
+  e.compute_us = k.busy_us ? k.busy_us(prob, dev.sm_count) : m.flops / rate;
   const double traffic = m.compulsory_bytes + (k.extra_traffic_bytes ? k.extra_traffic_bytes(prob) : 0.0);
   e.memory_us = traffic / (c.bw_gbs * 1e3 * hbm_eff);
   // resident workgroups overlap each other's set-up, so only the launch's first fill and last drain are exposed
-  e.launch_us = c.launch_overhead_us * std::max(k.launches, 1) + (fam ? fam->fill_us : 2.0);
+  e.launch_us = c.launch_overhead_us * std::max(k.launches, 1) +
+                (k.busy_us ? 0.0 : fam ? fam->fill_us : 2.0);
   {
     std::lock_guard<std::mutex> lock(g_scale_mu);
     const auto it = backend_scale().find(to_string(k.backend));

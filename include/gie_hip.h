@@ -26,6 +26,9 @@
  *   gie_hip_conv_stem, _stem_check   transposes + tcmma_kernel for the 7x7 stride-2 stem (in_channels <= 4), fused
  *   gie_hip_conv_narrow, _narrow_check transposes + tcmma_kernel (+ split-K reduce) for 3x3 layers with few pixels
  *                                                                         src/kernels/tensor_core_mma.cu:61-82,99-251,309-316
+ *   gie_hip_conv_mini, _mini_check   both transposes + tcmma_kernel + splitk_reduce (16-bit) and
+ *                                    implicit_gemm_kernel<<<>>> (FP32) for small layers, one launch
+ *                                                                         src/kernels/tensor_core_mma.cu:61-82,99-251,297-324
  *   gie_hip_conv_slab, _slab_check   both transposes + tcmma_kernel (split-K partials included) for 3x3 stride-1
  *                                    layers, fused: one launch straight from NCHW x / OIHW w
  *                                                                         src/kernels/tensor_core_mma.cu:61-82,99-251,297-324
@@ -222,6 +225,17 @@ int gie_hip_conv_stem(int dtype, const gie_conv_geom* g, const void* x, const vo
 int gie_hip_narrow_check(const gie_conv_geom* g, int* lds_bytes);
 int gie_hip_conv_narrow(int dtype, const gie_conv_geom* g, const void* x, const void* w, const void* bias, void* y,
                         void* stream);
+
+/* Small convolution straight from NCHW x and OIHW w, any filter of at most 64 taps, any stride, padding and channel
+   count, the whole reduction in one workgroup (one launch, no workspace): fused bias + ReLU, dtype GIE_HIP_FP32,
+   _FP16, _BF16 or _TF32 (float tensors, operands rounded to TF32 in the kernel). Every pointer needs only its
+   element's alignment; bias may be NULL. _config_get: tile side (filters and pixels per workgroup) and waves sharing the reduction; _check:
+   0 if configuration `config` takes the geometry (lds_bytes, optional: LDS per workgroup). */
+int gie_hip_mini_config_count(void);
+int gie_hip_mini_config_get(int config, int* tile, int* waves);
+int gie_hip_mini_check(int config, int dtype, const gie_conv_geom* g, int* lds_bytes);
+int gie_hip_conv_mini(int config, int dtype, const gie_conv_geom* g, const void* x, const void* w, const void* bias,
+                      void* y, void* stream);
 
 /* One registered slab configuration: tile_m (32) output channels x a slab of `rows` output rows of one image laid
    out `pitch` positions per row (in_w + 1 <= pitch), channel slices of tile_k, `stages` LDS load stages,

@@ -80,7 +80,9 @@ double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   if (waves_of(config) == 16) per_load *= !one && !nine ? 0.85 : k16 ? 1.0 : one ? 0.7 : 0.95;
   if (k16 && p.gemm_k() % 2 != 0) per_load *= 3.5;  // weights element by element (3x3, 331 channels: 44 us)
   const double share = std::max(1.0, double(blocks_of(config, prob)) / std::max(cus, 1));
-  return 0.5 + share * ((t == 16 ? 1.3 : 1.0) + loads * per_load);
+  // a CU with a single workgroup is bound by its latency, not by its load path (1024 -> 256, 196 pixels: 5.7 us)
+  if (k16 && one && t == 32) per_load -= 0.0038 * std::max(0.0, 2.0 - share);
+  return 0.5 + share * ((t == 16 ? 1.3 : 1.0) + loads * per_load) + (t == 16 ? 0.7 * (share - 1.0) : 0.0);
 }
 
 int mini_best_config(const ConvProblem& prob, int cus, double* us) {

@@ -22,6 +22,7 @@ void register_slab_family(std::vector<KernelDesc>& out);    // slab_family.cpp
 void register_stack_family(std::vector<KernelDesc>& out);   // stack_family.cpp
 void register_deep_family(std::vector<KernelDesc>& out);    // deep_family.cpp
 void register_mini_family(std::vector<KernelDesc>& out);    // mini_family.cpp
+void register_gather_family(std::vector<KernelDesc>& out);  // gather_family.cpp
 
 std::string KernelDesc::describe() const {
   std::ostringstream os;
@@ -47,6 +48,7 @@ std::vector<KernelDesc>& registry_storage() {
     register_stack_family(r);   // likewise
     register_deep_family(r);    // likewise
     register_mini_family(r);
+    register_gather_family(r);
     std::set<std::string> names;
     for (const auto& k : r) {
       if (!names.insert(k.name).second) throw Error(StatusCode::kInternal, "duplicate kernel name " + k.name);

@@ -216,6 +216,10 @@ _HIP = {
     "gie_hip_mini_config_get": ([_i, _ip, _ip], _i),
     "gie_hip_mini_check": ([_i, _i, _GP, _ip], _i),
     "gie_hip_conv_mini": ([_i, _i, _GP, _vp, _vp, _vp, _vp, _vp], _i),
+    "gie_hip_gather_config_count": ([], _i),
+    "gie_hip_gather_config_get": ([_i, _ip, _ip, _ip], _i),
+    "gie_hip_gather_check": ([_i, _GP, _ip], _i),
+    "gie_hip_conv_gather": ([_i, _i, _GP, _vp, _vp, _vp, _vp, _vp], _i),
     "gie_hip_slab_config_count": ([], _i),
     "gie_hip_slab_config_get": ([_i, ctypes.POINTER(GieSlabConfig)], _i),
     "gie_hip_slab_check": ([_i, _GP, _ip], _i),

@@ -29,6 +29,8 @@
  *   gie_hip_conv_mini, _mini_check   both transposes + tcmma_kernel + splitk_reduce (16-bit) and
  *                                    implicit_gemm_kernel<<<>>> (FP32) for small layers, one launch
  *                                                                         src/kernels/tensor_core_mma.cu:61-82,99-251,297-324
+ *   gie_hip_conv_gather, _gather_check  both transposes + tcmma_kernel, fused: one launch straight from NCHW / OIHW
+ *                                                                         src/kernels/tensor_core_mma.cu:61-82,99-251,297-324
  *   gie_hip_conv_slab, _slab_check   both transposes + tcmma_kernel (split-K partials included) for 3x3 stride-1
  *                                    layers, fused: one launch straight from NCHW x / OIHW w
  *                                                                         src/kernels/tensor_core_mma.cu:61-82,99-251,297-324
@@ -236,6 +238,17 @@ int gie_hip_mini_config_get(int config, int* tile, int* waves);
 int gie_hip_mini_check(int config, int dtype, const gie_conv_geom* g, int* lds_bytes);
 int gie_hip_conv_mini(int config, int dtype, const gie_conv_geom* g, const void* x, const void* w, const void* bias,
                       void* y, void* stream);
+
+/* Pointwise convolution (1x1 filter) of any stride, padding and image size straight from NCHW x and OIHW w, the
+   activation tile gathered by the kernel (one launch, no workspace): fused bias + ReLU, dtype GIE_HIP_FP16 / _BF16, an
+   even channel count and w 4-byte aligned (GIE_HIP_EUNSUPPORTED otherwise), the other pointers 2-byte aligned; bias may
+   be NULL. _config_get: filters x pixels per workgroup and its threads; _check: 0 if configuration `config` takes the
+   geometry (lds_bytes, optional: LDS per workgroup). */
+int gie_hip_gather_config_count(void);
+int gie_hip_gather_config_get(int config, int* tile_m, int* tile_n, int* threads);
+int gie_hip_gather_check(int config, const gie_conv_geom* g, int* lds_bytes);
+int gie_hip_conv_gather(int config, int dtype, const gie_conv_geom* g, const void* x, const void* w, const void* bias,
+                        void* y, void* stream);
 
 /* One registered slab configuration: tile_m (32) output channels x a slab of `rows` output rows of one image laid
    out `pitch` positions per row (in_w + 1 <= pitch), channel slices of tile_k, `stages` LDS load stages,

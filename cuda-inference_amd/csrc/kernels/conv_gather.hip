@@ -22,7 +22,7 @@
 // one image: 49.0 -> 31.7; 896 -> 448 over 10x10, batch 41: 22.0 -> 13.8.
 #include <algorithm>
 
-#include "device_common.h"
+#include "tile_epilogue.h"
 
 namespace gie_hip {
 namespace {
@@ -208,59 +208,8 @@ __global__ __launch_bounds__(WO * WP * 64) void gather_kernel(const uint16_t* __
     }
   }
 
-  // ---- epilogue: bias + ReLU + one rounding into [filter][pixel] rows, then whole rows of y ----
-  constexpr int YROW = TP * 2 + 16;
-#pragma unroll
-  for (int j = 0; j < FO; ++j) {
-    const int oc = wo * WTO + j * 32 + fr;
-    const float bv = bias != nullptr && o0 + oc < g.O ? E::to_f32(bias[o0 + oc]) : 0.0f;
-#pragma unroll
-    for (int i = 0; i < FP; ++i) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = acc[i][j][4 * q + e] + bv;
-          if (g.relu) v[e] = fmaxf(v[e], 0.0f);
-        }
-        const int px = wp * WTP + i * 32 + 8 * q + 4 * fc;  // four consecutive pixels
-        *reinterpret_cast<u32x2*>(ga_lds + oc * YROW + px * 2) = u32x2{E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
-      }
-    }
-  }
-  __syncthreads();
-  constexpr int CK = TP / 8, RPP = NT / CK;  // 16-byte chunks per row, rows per pass
-  static_assert(NT % CK == 0, "a thread keeps its chunk column");
-  const int ck = tid % CK, r0 = tid / CK;
-  const int nn = n0 + ck * 8, b0 = nn / g.OHW, p0 = nn - b0 * g.OHW;
-  const bool whole = nn + 8 <= g.N && p0 + 8 <= g.OHW;  // the eight pixels lie in one image
-  uint16_t* const y0 = y + static_cast<long long>(b0) * g.O * g.OHW + p0;
-  constexpr int NP = TO / RPP;  // passes over the tile's rows
-  static_assert(NP * RPP == TO, "whole passes");
-  if (whole) {
-#pragma unroll
-    for (int q = 0; q < NP; ++q) {
-      const int r = r0 + q * RPP;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(ga_lds + r * YROW + ck * 16);
-      if (o0 + r < g.O) __builtin_memcpy(y0 + static_cast<long long>(o0 + r) * g.OHW, &v, 16);
-    }
-    return;
-  }
-  for (int r = r0; r < TO && o0 + r < g.O; r += RPP) {
-    const u32x4 v = *reinterpret_cast<const u32x4*>(ga_lds + r * YROW + ck * 16);
-    uint16_t* d = y0 + static_cast<long long>(o0 + r) * g.OHW;
-    int pp = p0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      if (nn + q < g.N) *d = uint16_t(v[q >> 1] >> (16 * (q & 1)));
-      ++d;
-      if (++pp == g.OHW) {  // on to the same filter of the next image
-        pp = 0;
-        d += static_cast<long long>(g.O - 1) * g.OHW;
-      }
-    }
-  }
+  // ---- every wave has finished its last step (the barrier above): the stages become the output tile ----
+  tile_to_y<E, TO, TP, WO, WP>(acc, ga_lds, bias, y, tid, o0, n0, g.O, g.OHW, g.N, g.relu);
 }
 
 // ---- configurations: filters x pixels of the tile, threads ----

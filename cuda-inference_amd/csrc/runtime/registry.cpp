@@ -23,6 +23,7 @@ void register_stack_family(std::vector<KernelDesc>& out);   // stack_family.cpp
 void register_deep_family(std::vector<KernelDesc>& out);    // deep_family.cpp
 void register_mini_family(std::vector<KernelDesc>& out);    // mini_family.cpp
 void register_gather_family(std::vector<KernelDesc>& out);  // gather_family.cpp
+void register_nhwc_family(std::vector<KernelDesc>& out);    // nhwc_family.cpp
 
 std::string KernelDesc::describe() const {
   std::ostringstream os;
@@ -49,6 +50,7 @@ std::vector<KernelDesc>& registry_storage() {
     register_deep_family(r);    // likewise
     register_mini_family(r);
     register_gather_family(r);
+    register_nhwc_family(r);
     std::set<std::string> names;
     for (const auto& k : r) {
       if (!names.insert(k.name).second) throw Error(StatusCode::kInternal, "duplicate kernel name " + k.name);

@@ -93,7 +93,9 @@ struct Fns {
     const int64_t hw = int64_t(p.in_h) * p.in_w;
     const bool flat = p.stride_h == 1 && p.stride_w == 1 && p.pad_h == 0 && p.pad_w == 0;
     const int px = std::min(flat && hw % 4 == 0 ? 4 : flat && hw % 2 == 0 ? 2 : 1, t.m == 256 ? 2 : 4);
-    const double loads = (double(t.n) / px + t.m / 8.0) * 16.0 / 2400.0;  // us of a step's vector loads
+    // a strided row of x takes twice the cache lines (256 -> 512, 56x56 /2, batch 32: 38 us at 128x128)
+    const double spread = p.stride_w > 1 ? 1.35 : 1.0;
+    const double loads = (spread * double(t.n) / px + t.m / 8.0) * 16.0 / 2400.0;  // us of a step's vector loads
     const double steps = double((p.in_channels + 63) / 64), share = double(blocks(prob)) / std::max(cus, 1);
     return f.fixed + std::max(steps * (f.alone + f.alone_load * loads),
                               share * (f.start + steps * (f.step + f.step_load * loads)));

@@ -125,6 +125,27 @@ struct Fns {
     const size_t l = lds(prob);
     return l > 80 * 1024 ? 1 : 2;
   }
+  // Fixed cost, the repack at `traffic` us/MB, a CU's share of the workgroups at a start-up cost and a cost for each
+  // 32-channel slice (or one workgroup's latency), output stores, and the reduce. Fitted to 20-125 layers per tile on one
+  // MI355X (7-12 % rms); a FLOP rate missed by up to 2x on images of 20 and more a side with few channels.
+  static double busy_us(const ConvProblem& prob, int cus) {
+    struct Fit {
+      double fixed, alone, alone_slice, start, slice, out, reduce, traffic;
+    };
+    const Entry& en = e();
+    const Fit f = en.info.kernel_h > 1 ? en.info.stages == 2 ? Fit{4.9, 1.8, 0.98, 5.3, 0.92, 0.59, 0.31, 0.57}
+                                                             : Fit{5.9, 1.8, 0.45, 2.7, 0.58, 0.0, 0.49, 0.97}
+                  : en.info.tile_m == 64 ? Fit{6.4, 0.0, 0.24, 1.4, 0.18, 0.68, 0.31, 0.39}
+                                         : Fit{8.6, 0.7, 0.37, 6.9, 0.21, 0.43, 0.25, 0.28};
+    const double slices = double(slices_of(prob, en)) / en.split;
+    const double share = double(blocks(prob)) / std::max(cus, 1);
+    const double y = double(prob.p.output_shape().numel()) / 1e6;  // million outputs
+    const double moved = (double(prob.p.batch) * prob.p.in_h * prob.p.in_w +
+                          double(prob.p.out_channels) * prob.p.kernel_h * prob.p.kernel_w) * c_pad_of(prob) * 4.0 / 1e6;
+    const double reduce = en.split > 1 ? (en.split + 1) * 4.0 * y * f.reduce : 0.0;
+    return f.fixed + moved * f.traffic + y * f.out + reduce +
+           std::max(f.alone + f.alone_slice * slices, share * (f.start + f.slice * slices));
+  }
   static void launch(const LaunchArgs& la) {
     const Entry& en = e();
     const ConvProblem& prob = *la.problem;
@@ -168,6 +189,7 @@ void fill_fns(int idx, KernelDesc& k) {
       k.num_blocks = &Fns<I>::blocks;
       k.extra_traffic_bytes = &Fns<I>::extra_traffic;
       k.blocks_per_cu = &Fns<I>::occupancy;
+      k.busy_us = &Fns<I>::busy_us;
       k.launch = &Fns<I>::launch;
       return;
     }

@@ -118,6 +118,11 @@ struct Fns {
     (void)xw;  // read once by the repack: part of the compulsory traffic already
     return 2.0 * xwp + part;
   }
+  // The repack runs before the GEMM and does not overlap it: x read and its padded copy written at copy rate.
+  static double serial_us(const ConvProblem& prob) {
+    const Conv2DParams& p = prob.p;
+    return double(p.batch) * p.in_h * p.in_w * (p.in_channels + c_pad_of(prob)) * 2.0 / 4.3e6;
+  }
   static int occupancy(const ConvProblem& prob) {
     int n = 1;
     if (gie_hip_igemm_occupancy(e().config, dtype_of(prob.precision), &n) != GIE_HIP_OK) {
@@ -169,6 +174,7 @@ struct FnTable {
     k.num_blocks = &Fns<I>::blocks;
     k.extra_traffic_bytes = &Fns<I>::extra_traffic;
     k.blocks_per_cu = &Fns<I>::occupancy;
+    k.serial_us = &Fns<I>::serial_us;
     k.launch = &Fns<I>::launch;
   }
 };
@@ -223,6 +229,9 @@ void register_mfma_family(std::vector<KernelDesc>& out) {
     k.tile_k = en.info.tile_k;
     k.uses_tensor_cores = true;
     k.launches = 2 + (en.split > 1 ? 1 : 0);
+    // four waves on a tile of 64 x 128 and more reach 0.65 of the eight-wave tiles' rate (BF16 3x3 64 -> 64, 56x56,
+    // batch 32: 39.5 us where 64x128x64_w2x4 takes 31)
+    if (en.info.threads <= 256 && en.info.tile_m * en.info.tile_n >= 64 * 128) k.relative_rate = 0.65;
     fill_fns<0>(int(i), k);
     out.push_back(std::move(k));
   }

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <string>
 #include <vector>
 
@@ -76,13 +77,19 @@ double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   // operand loads of a lane over the reduction's whole supersteps (3x3: 9 chunks of each lane group, else 64 k)
   const int64_t ss = nine ? 9 * (64 / t) * ck : 8 * ck;
   const double loads = double((p.gemm_k() + ss - 1) / ss * ss) / (ck * (64 / t)) * (ck + 1);
-  double per_load = !one && !nine ? (t == 16 ? 0.03 : 0.022) : !k16 ? 0.012 : t == 16 && one ? 0.0057 : 0.0085;
-  if (waves_of(config) == 16) per_load *= !one && !nine ? 0.85 : k16 ? 1.0 : one ? 0.7 : 0.95;
-  if (k16 && p.gemm_k() % 2 != 0) per_load *= 3.5;  // weights element by element (3x3, 331 channels: 44 us)
-  const double share = std::max(1.0, double(blocks_of(config, prob)) / std::max(cus, 1));
+  double per_load = !one && !nine ? (t == 16 ? 0.014 : 0.022) : !k16 ? 0.012 : t == 16 && one ? 0.0057 : 0.0085;
+  const double wave = std::max(1.0, double(blocks_of(config, prob)) / std::max(cus, 1));
+  if (waves_of(config) == 16 && (one || nine || wave <= 1.0))
+    per_load *= !one && !nine ? 0.85 : k16 ? 1.0 : one ? 0.7 : 0.95;
+  // weights element by element (3x3, 331 channels: 44 us)
+  if (k16 && p.gemm_k() % 2 != 0) per_load *= one || nine ? 3.5 : 1.4;
+  // strided rows of x take twice the cache lines (1x1 544 -> 32, 29x29 /2, batch 53: 37 us at 16x16)
+  if (k16 && (one || nine) && p.stride_w > 1 && wave > 1.0) per_load *= 1.6;
+  const double share = k16 ? 0.5 * (wave + std::ceil(wave)) : wave;  // the last wave of workgroups is partly empty
   // a CU with a single workgroup is bound by its latency, not by its load path (1024 -> 256, 196 pixels: 5.7 us)
   if (k16 && one && t == 32) per_load -= 0.0038 * std::max(0.0, 2.0 - share);
-  return 0.5 + share * ((t == 16 ? 1.3 : 1.0) + loads * per_load) + (t == 16 ? 0.7 * (share - 1.0) : 0.0);
+  const double start = t != 16 ? 1.0 : k16 && one ? 0.7 : 1.3;
+  return 0.5 + share * (start + loads * per_load) + (t == 16 ? 0.7 * (share - 1.0) : 0.0);
 }
 
 int mini_best_config(const ConvProblem& prob, int cus, double* us) {

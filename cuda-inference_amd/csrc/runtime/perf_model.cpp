@@ -5,7 +5,8 @@
 //   compute = FLOPs / (MFMA peak x family MFMA efficiency x tile efficiency x wave efficiency)
 //   memory  = (compulsory bytes + the kernel's extra traffic) / (HBM bandwidth x family HBM efficiency)
 //   fixed   = launches x dispatch cost + the family's cost of filling and draining a launch
-//   time    = max(compute, memory) + fixed      (reported as launch_us; "launch"-bound when it dominates)
+//   serial  = passes that do not overlap the main kernel (KernelDesc::serial_us: a repack, a reduce)
+//   time    = max(compute, memory) + fixed + serial  (reported as launch_us; "launch"-bound when it dominates)
 // A family with a formula of its own (KernelDesc::busy_us: everything but dispatch) takes that as its compute time.
 // * Family efficiencies are not guesses per backend: each is what that kernel family reached on an MI355X in the
 //   library's benchmark protocol (per-call time, inputs resident in HBM), listed in kFamilies with the measurement.
@@ -55,7 +56,7 @@ struct FamilyProfile {
 // efficiency alone carries the measurement.
 constexpr FamilyProfile kFamilies[] = {
     {"slab_", 0.66, 0.45, 2.5},     // L2 9.1 us (split form: steps at 0.66 of peak, ~3.7 us of set-up, first slice
-                                    // and epilogue per unit); the other forms share the profile and the tuner
+                                    // and epilogue per unit); the other forms' rates are relative to it
     {"band_", 0.27, 0.45, 5.0},     // L2 18.9 us including the weight repack launch
     {"halo_", 0.37, 0.40, 10.0},    // L2 23.3 us including the repack launch, L5 24.7 us at split 4
     {"mfma_", 0.22, 0.35, 8.0},     // L2 25.7 us, L3 87 us, L4 145 us, L5 26.0 us at split 4
@@ -66,6 +67,10 @@ constexpr FamilyProfile kFamilies[] = {
     {"stack_", 0.33, 0.40, 4.1},    // L5 9.6 us at split 2 (6.7 conv + 2.8 reduce), 10.2 at split 1
     {"deep_", 0.44, 0.40, 2.9},     // L5 6.6 us: steps at 0.44 of peak, ~4.2 us of set-up, first stage and
                                     // partial-tile exchange per unit
+    // families with a formula of their own: only the bandwidth is used
+    {"mini_", 0.30, 0.50, 0.0},     // its cases are far below the bandwidth
+    {"nhwc_", 0.30, 0.50, 0.0},     // BF16 3x3 64 -> 64, 56x56, batch 32: 28.7 us = 2.7 TB/s with the repack's copy
+    {"gather_", 0.30, 0.50, 0.0},   // 1x1 256 -> 128, 56x56, batch 32: 23.2 us = 3.3 TB/s; at /2 to 512: 2.7 TB/s
     {"f32_", 0.30, 0.35, 2.0},      // FP32 / TF32 vector kernels: not benchmarked, assumed
 };
 
@@ -298,7 +303,7 @@ Estimate estimate_kernel(const ConvProblem& prob, const KernelDesc& k, const Dev
   e.wave_efficiency = double(blocks) / double(waves * slots * xcds);
 
   const double peak_tflops = k.uses_tensor_cores ? c.fp16_tc_tflops : c.fp32_tflops;
-  const double rate = peak_tflops * 1e6 * mfma_eff * std::max(e.tile_efficiency, 1e-3) *
+  const double rate = peak_tflops * 1e6 * mfma_eff * k.relative_rate * std::max(e.tile_efficiency, 1e-3) *
                       std::max(e.wave_efficiency, 1e-3);  // FLOP per us
   e.compute_us = k.busy_us ? k.busy_us(prob, dev.sm_count) : m.flops / rate;
   const double traffic = m.compulsory_bytes + (k.extra_traffic_bytes ? k.extra_traffic_bytes(prob) : 0.0);
@@ -315,7 +320,7 @@ Estimate estimate_kernel(const ConvProblem& prob, const KernelDesc& k, const Dev
     }
   }
   e.bound = bound_of(e.compute_us, e.memory_us, e.launch_us);
-  e.time_us = std::max(e.compute_us, e.memory_us) + e.launch_us;
+  e.time_us = std::max(e.compute_us, e.memory_us) + e.launch_us + (k.serial_us ? k.serial_us(prob) : 0.0);
   return e;
 }
 

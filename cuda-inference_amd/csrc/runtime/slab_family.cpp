@@ -67,6 +67,26 @@ int slices_of(const ConvProblem& prob, const Entry& en) {
   return (prob.p.in_channels + en.info.tile_k - 1) / en.info.tile_k;
 }
 
+// The configuration with en's rows and pitch in the full form, -1 if there is none or en is that form.
+int full_form_of(const Entry& en) {
+  if (en.info.form == 0) return -1;
+  int best = -1;
+  for (const Entry& o : entries())
+    if (o.info.form == 0 && o.info.rows == en.info.rows && o.info.pitch == en.info.pitch &&
+        o.info.tile_k == en.info.tile_k && (best < 0 || o.config < best))
+      best = o.config;
+  return best;
+}
+
+// Steady-state rate of each form against the split form's, whose profile the family carries (MI355X, FP16 3x3 256 -> 256
+// over 14x14, batch 32 / 288 -> 367 over 12x12, batch 22: split 9.1 / 15.6 us, pipelined 10.3 / 17.7, two lean
+// workgroups a CU 15.1 / 19.8, full 16.0 / 28.8). Taking them for equal made the dispatcher choose the full form.
+double rate_of(const gie_slab_config& info) {
+  if (info.form == 3) return 1.0;
+  if (info.form == 2) return 0.82;
+  return info.workgroups_per_cu > 1 ? 0.95 : 0.46;
+}
+
 template <int I>
 struct Fns {
   static const Entry& e() { return entries()[I]; }
@@ -128,6 +148,11 @@ struct Fns {
     const double c = double(p.in_channels) / double(((p.in_channels + 31) / 32) * 32);
     return std::min(1.0, pos) * o * c;
   }
+  // The reduce follows the convolution instead of overlapping it (288 -> 367 over 12x12, batch 22, split form: split 2
+  // takes 21.5 us, split 1 15.6), at about 2.2 TB/s of partials read and output written as FP32.
+  static double serial_us(const ConvProblem& prob) {
+    return e().split > 1 ? (e().split + 1) * double(prob.p.output_shape().numel()) * 4.0 / 2.2e6 : 0.0;
+  }
   static void launch(const LaunchArgs& la) {
     const Entry& en = e();
     const ConvProblem& prob = *la.problem;
@@ -142,7 +167,12 @@ struct Fns {
       return;
     }
     if (stage(1)) {
-      const int rc = gie_hip_conv_slab(en.config, dt, &g, la.x, la.w, la.bias, la.y, part, en.split, la.stream);
+      int rc = gie_hip_conv_slab(en.config, dt, &g, la.x, la.w, la.bias, la.y, part, en.split, la.stream);
+      if (rc == GIE_HIP_EUNSUPPORTED) {
+        // the full form of the same rows also takes an x aligned to 2 bytes only; its split-K partials are the same
+        const int full = full_form_of(en);
+        if (full >= 0) rc = gie_hip_conv_slab(full, dt, &g, la.x, la.w, la.bias, la.y, part, en.split, la.stream);
+      }
       if (rc == GIE_HIP_EUNSUPPORTED) {
         fallback_of(en.precision).launch(la);
         return;
@@ -169,6 +199,7 @@ void fill_fns(int idx, KernelDesc& k) {
       k.extra_traffic_bytes = &Fns<I>::extra_traffic;
       k.blocks_per_cu = &Fns<I>::occupancy;
       k.tile_efficiency = &Fns<I>::tile_efficiency;
+      k.serial_us = &Fns<I>::serial_us;
       k.launch = &Fns<I>::launch;
       return;
     }
@@ -211,6 +242,7 @@ void register_slab_family(std::vector<KernelDesc>& out) {
     k.tile_k = en.info.tile_k * 9;
     k.uses_tensor_cores = true;
     k.launches = 1 + (en.split > 1 ? 1 : 0);
+    k.relative_rate = rate_of(en.info);
     fill_fns<0>(int(i), k);
     out.push_back(std::move(k));
   }

@@ -73,6 +73,10 @@ struct KernelDesc {
   // Modeled time (us) of the main kernel on `cus` CUs beyond its dispatch, for a family whose time follows a formula of
   // its own; the cost model takes it in place of FLOPs over a rate (MI355X-specific addition; null -> FLOP rate).
   double (*busy_us)(const ConvProblem&, int cus) = nullptr;
+  // Modeled time (us) of passes before or after the main kernel that do not overlap it (MI355X-specific addition).
+  double (*serial_us)(const ConvProblem&) = nullptr;
+  // This entry's compute rate relative to its family's profile (MI355X-specific addition).
+  double relative_rate = 1.0;
 
   std::string describe() const;
 };

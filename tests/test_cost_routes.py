@@ -1,0 +1,42 @@
+"""The cost model's order inside and between families where measurements separate them (no GPU needed): each case names
+the entry or family that was measured faster and the one it must stay ahead of."""
+import pytest
+
+import gie
+
+P = gie.Problem
+
+
+def _us(p):
+    return dict(gie.model_rank(p))
+
+
+@pytest.mark.parametrize("p,first,second", [
+    # the split form of a 14-row slab beats the full form of the same slab: 9.1 and 16.0 us
+    (P(32, 256, 14, 14, 256, 3, 3, 1, 1, 1, 1, precision="fp16"), "slab_fp16_3x3_32x14r16_k32_s3_ld_sk1",
+     "slab_fp16_3x3_32x14r16_k32_s3_sk1"),
+    # a reduce over 1.2 million outputs costs more than split-K gains: 15.6 and 21.5 us
+    (P(22, 288, 12, 12, 367, 3, 3, 1, 1, 1, 1, precision="fp16"), "slab_fp16_3x3_32x14r16_k32_s3_ld_sk1",
+     "slab_fp16_3x3_32x14r16_k32_s3_ld_sk2"),
+    # 56-pixel rows leave a 64-position band's stores short: 28.7 and 56.5 us; halo 48.3
+    (P(32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_64x128x64_sk1",
+     "band_bf16_3x3_32x256x32_s3_sk1"),
+    (P(32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_64x128x64_sk1",
+     "halo_bf16_3x3_64x128x32_s2_sk1"),
+    # strided rows of x: 28.7 and 38.0 us
+    (P(32, 256, 56, 56, 512, 1, 1, 2, 2, 0, 0, precision="fp16"), "gather_fp16_1x1_256x128_t512",
+     "gather_fp16_1x1_128x128_t256"),
+    (P(53, 544, 29, 29, 32, 1, 1, 2, 2, 0, 0, precision="bf16"), "mini_bf16_32x32_k16w", "mini_bf16_16x16_k8w"),
+])
+def test_measured_order(p, first, second):
+    us = _us(p)
+    assert us[first] < us[second], (us[first], us[second])
+
+
+@pytest.mark.parametrize("prec", ["fp32", "tf32", "fp16", "bf16"])
+def test_every_estimate_is_finite_and_positive(prec):
+    for p in (P(1, 8, 1, 1, 8, 1, 1, 1, 1, 0, 0, precision=prec), P(3, 7, 33, 31, 9, 3, 3, 2, 1, 0, 2, precision=prec),
+              P(64, 2048, 56, 56, 2048, 3, 3, 1, 1, 1, 1, precision=prec),
+              P(2, 5, 40, 3, 6, 11, 3, 3, 3, 5, 1, precision=prec)):
+        us = gie.model_rank(p)
+        assert us and all(0.0 < u < 1e7 for _, u in us), us[:3]

@@ -31,6 +31,33 @@
 namespace gie_hip {
 namespace {
 
+// FP32 (v_mfma_f32_32x32x2_f32): the same kernel on twice the 16-bit units, a 16-byte fragment being four channels and
+// so four MFMAs, each with an accumulator of its own: no MFMA waits for the one before. Every 16 steps (512 channels) the
+// four are added into the tile's sums, so that no sum runs over more than 128 products and the error does not grow with
+// the reduction (3x3 512 channels: 1.4e-7 of the norm, 4.0e-7 for one chain). Here the matrix cores bound: a step runs at
+// 0.81 (64 x 64) and 0.88 (128 x 128) of their rate, the rest is the last round of tiles and the repack. Measured: 3x3
+// 128 -> 128 over 28x28, batch 32: 118 -> 92 us; 64 -> 64 over 56x56, batch 32: 148 -> 97; 7x7 stride 2 3 -> 64 over
+// 224x224, batch 8: 119 -> 50.
+struct NhF32 {
+  static constexpr int kDtype = GIE_HIP_FP32, kAcc = 4;
+  template <int N>
+  static __device__ __forceinline__ void mma(u32x4 a, u32x4 b, f32x16 (&c)[N]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      c[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(f32x4, a)[e], __builtin_bit_cast(f32x4, b)[e], c[e],
+                                                  0, 0, 0);
+  }
+};
+template <typename E16>
+struct NhHalf : E16 {
+  static constexpr int kAcc = 1;
+  template <int N>
+  static __device__ __forceinline__ void mma(u32x4 a, u32x4 b, f32x16 (&c)[N]) {
+    c[0] = E16::mfma32(a, b, c[0]);
+  }
+};
+
+// Cp, Kp and the 64-unit steps count 16-bit units: an FP32 channel is two.
 struct NhwcGeom {
   int C, H, W, O, KH, KW, SH, SW, PH, PW, OW, OHW, N;
   int Cp, Hp, Wp;
@@ -46,16 +73,17 @@ struct NhwcGeom {
 
 // ---- repack ----
 constexpr int kNhThreads = 256;
-constexpr int kNhFilter = 16384;  // elements of a filter staged in LDS
+constexpr int kNhFilter = 32768;  // bytes of a filter staged in LDS
 
-struct NhwcRepack {
-  const uint16_t* x;
-  const uint16_t* w;
-  uint16_t* xp;
-  uint16_t* wp;
+template <typename T>
+struct NhwcRepack {  // Cp, Kp and run in elements
+  const T* x;
+  const T* w;
+  T* xp;
+  T* wp;
   int B, C, H, W, HW, Cp, Hp, Wp, PH, PW, O, KH, KW, Kp, run;  // run: elements per filter row, padded
-  int gpi, cgs;           // four-pixel groups per image rounded up to 16, 32-channel groups
-  long long x_waves;      // wave items: (image, 16 groups, 32 channels)
+  int gpi, cgs;           // four-pixel groups per image rounded up to 16, groups of four 16-byte chunks of channels
+  long long x_waves;      // wave items: (image, 16 pixel groups, channel group)
   long long x_blocks, border, b_blocks;  // border: 16-byte chunks of padding
 };
 
@@ -72,25 +100,37 @@ __device__ __forceinline__ u32x2 nh_load4(const uint16_t* p, int left) {
   }
   return v;
 }
+__device__ __forceinline__ u32x4 nh_load4(const uint32_t* p, int left) {
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (left >= 4) {
+    __builtin_memcpy(&v, p, 16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] = i < left ? p[i] : 0u;
+  }
+  return v;
+}
 
-__global__ __launch_bounds__(kNhThreads) void nhwc_repack_kernel(NhwcRepack j) {
-  __shared__ __attribute__((aligned(16))) uint16_t buf[kNhFilter];
+template <typename T>
+__global__ __launch_bounds__(kNhThreads) void nhwc_repack_kernel(NhwcRepack<T> j) {
+  constexpr int CH = 16 / int(sizeof(T)), FL = kNhFilter / int(sizeof(T));  // channels of a 16-byte chunk, staged elements
+  __shared__ __attribute__((aligned(16))) T buf[FL];
   const int tid = threadIdx.x, lane = tid & 63;
   long long blk = blockIdx.x;
   if (blk < j.x_blocks) {
-    // a wave: 16 lanes along pixels (4 each) x 4 lane groups along channels (8 each)
+    // a wave: 16 lanes along pixels (4 each) x 4 lane groups along channels (CH each)
     const long long item = blk * (kNhThreads / 64) + (tid >> 6);
     if (item >= j.x_waves) return;
     const int cg = int(item % j.cgs);
     const long long rest = item / j.cgs;
     const int per = j.gpi / 16, b = int(rest / per), p = (int(rest - static_cast<long long>(b) * per) * 16 + (lane & 15)) * 4;
-    const int c8 = cg * 32 + (lane >> 4) * 8;
+    const int c8 = (cg * 4 + (lane >> 4)) * CH;
     if (p >= j.HW || c8 >= j.Cp) return;
-    const uint16_t* src = j.x + (static_cast<long long>(b) * j.C + c8) * j.HW + p;
-    u32x2 in[8];
+    const T* src = j.x + (static_cast<long long>(b) * j.C + c8) * j.HW + p;
+    decltype(nh_load4(src, 0)) in[CH];
 #pragma unroll
-    for (int r = 0; r < 8; ++r)
-      in[r] = c8 + r < j.C ? nh_load4(src + static_cast<long long>(r) * j.HW, j.HW - p) : u32x2{0u, 0u};
+    for (int r = 0; r < CH; ++r)
+      in[r] = nh_load4(src + static_cast<long long>(r) * j.HW, c8 + r < j.C ? j.HW - p : 0);
     int h = p / j.W, w = p - h * j.W;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -98,7 +138,9 @@ __global__ __launch_bounds__(kNhThreads) void nhwc_repack_kernel(NhwcRepack j) {
         u32x4 v;
 #pragma unroll
         for (int d = 0; d < 4; ++d)
-          v[d] = __builtin_amdgcn_perm(in[2 * d + 1][q >> 1], in[2 * d][q >> 1], q & 1 ? 0x07060302u : 0x05040100u);
+          v[d] = CH == 4 ? in[d][q]
+                         : __builtin_amdgcn_perm(in[(2 * d + 1) % CH][q >> 1], in[(2 * d) % CH][q >> 1],
+                                                 q & 1 ? 0x07060302u : 0x05040100u);
         const long long px = (static_cast<long long>(b) * j.Hp + h + j.PH) * j.Wp + w + j.PW;
         *reinterpret_cast<u32x4*>(j.xp + px * j.Cp + c8) = v;
       }
@@ -111,7 +153,7 @@ __global__ __launch_bounds__(kNhThreads) void nhwc_repack_kernel(NhwcRepack j) {
     // padding: rows above, rows below, then the columns left and right of each image row
     const long long i = blk * kNhThreads + tid;
     if (i >= j.border) return;
-    const int cv = j.Cp / 8, c8 = int(i % cv) * 8;
+    const int cv = j.Cp / CH, c8 = int(i % cv) * CH;
     const long long cell = i / cv;
     const int top = j.PH * j.Wp, side = j.Wp - j.W, per = 2 * top + j.H * side;
     const int b = int(cell / per), e = int(cell - static_cast<long long>(b) * per);
@@ -130,35 +172,36 @@ __global__ __launch_bounds__(kNhThreads) void nhwc_repack_kernel(NhwcRepack j) {
   }
   // weights: one filter per workgroup, through LDS where it fits
   const int o = int(blk - j.b_blocks), rs = j.KH * j.KW, n = j.C * rs;
-  const uint16_t* src = j.w + static_cast<long long>(o) * n;
-  const bool staged = n <= kNhFilter;
+  const T* src = j.w + static_cast<long long>(o) * n;
+  const bool staged = n <= FL;
   if (staged) {
-    const int n8 = n & ~7;
-    for (int i = tid * 8; i < n8; i += kNhThreads * 8) __builtin_memcpy(buf + i, src + i, 16);
+    const int n8 = n & ~(CH - 1);
+    for (int i = tid * CH; i < n8; i += kNhThreads * CH) __builtin_memcpy(buf + i, src + i, 16);
     for (int i = n8 + tid; i < n; i += kNhThreads) buf[i] = src[i];
     __syncthreads();
   }
-  uint16_t* dst = j.wp + static_cast<long long>(o) * j.Kp;
-  for (int t = tid; t < j.Kp / 8; t += kNhThreads) {
-    const int r = (t * 8) / j.run, k = t * 8 - r * j.run, s = k / j.Cp, c8 = k - s * j.Cp;
+  T* dst = j.wp + static_cast<long long>(o) * j.Kp;
+  for (int t = tid; t < j.Kp / CH; t += kNhThreads) {
+    const int r = (t * CH) / j.run, k = t * CH - r * j.run, s = k / j.Cp, c8 = k - s * j.Cp;
     u32x4 v = {0u, 0u, 0u, 0u};
     if (s < j.KW) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
+      for (int q = 0; q < CH; ++q) {
         const int c = c8 + q, at = c * rs + r * j.KW + s;
         const uint32_t e = c < j.C ? (staged ? buf[at] : src[at]) : 0u;
-        v[q >> 1] |= e << (16 * (q & 1));
+        if (CH == 4) v[q % 4] = e;
+        else v[q / 2] |= e << (16 * (q & 1));
       }
     }
-    *reinterpret_cast<u32x4*>(dst + t * 8) = v;
+    *reinterpret_cast<u32x4*>(dst + t * CH) = v;
   }
 }
 
 // ---- GEMM ----
 template <typename E, int TO, int TP, int WO, int WP, int NST>
-__global__ __launch_bounds__(WO * WP * 64) void nhwc_kernel(const uint16_t* __restrict__ xp, const uint16_t* __restrict__ wk,
-                                                            const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-                                                            float* __restrict__ partial, NhwcGeom g) {
+__global__ __launch_bounds__(WO * WP * 64, E::kAcc == 4 && TO == 64 ? 3 : 1)
+void nhwc_kernel(const uint16_t* __restrict__ xp, const uint16_t* __restrict__ wk, const void* __restrict__ bias,
+                 void* __restrict__ y, float* __restrict__ partial, NhwcGeom g) {
   constexpr int NW = WO * WP, ROWB = 128, STG = (TO + TP) * ROWB;
   constexpr int LX = TP / 8 / NW, LW = TO / 8 / NW, NI = LX + LW;  // direct loads (8 rows each) per wave and step
   constexpr int WTP = TP / WP, WTO = TO / WO, FP = WTP / 32, FO = WTO / 32;
@@ -217,15 +260,34 @@ __global__ __launch_bounds__(WO * WP * 64) void nhwc_kernel(const uint16_t* __re
   // operands: A = pixels (rows), B = filters (columns); lane: row lane % 32, k-chunk 2 kk + lane / 32
   const int fr = lane & 31, fc = lane >> 5, swz = (fr >> 1) & 7;
   const unsigned a_row = unsigned((wp * WTP + fr) * ROWB), b_row = unsigned((TP + wo * WTO + fr) * ROWB);
+  constexpr int NA = E::kAcc;
+  f32x16 sum[FP][FO][NA];
+#pragma unroll
+  for (int i = 0; i < FP; ++i)
+#pragma unroll
+    for (int j = 0; j < FO; ++j)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) sum[i][j][a] = f32x16{};
+
+  // Fragments of 16-element step kk + 1 are read while step kk multiplies, across steps too: the last kk of a step meets
+  // the barrier first (the next step has landed for every wave, and every wave has read the last of this step's stage,
+  // which the loads of step t + NST then take) and reads the next step's first fragments before its own MFMAs.
   f32x16 acc[FP][FO];
 #pragma unroll
   for (int i = 0; i < FP; ++i)
 #pragma unroll
     for (int j = 0; j < FO; ++j) acc[i][j] = f32x16{};
-
-  // Fragments of 16-element step kk + 1 are read while step kk multiplies, across steps too: the last kk of a step meets
-  // the barrier first (the next step has landed for every wave, and every wave has read the last of this step's stage,
-  // which the loads of step t + NST then take) and reads the next step's first fragments before its own MFMAs.
+  auto add_up = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < FP; ++i)
+#pragma unroll
+      for (int j = 0; j < FO; ++j) {
+        if constexpr (NA == 4) acc[i][j] += (sum[i][j][0] + sum[i][j][1]) + (sum[i][j][2] + sum[i][j][3]);
+        else acc[i][j] = sum[i][j][0];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) sum[i][j][a] = f32x16{};
+      }
+  };
   u32x4 af[2][FP], bf[2][FO];
   auto rd = [&](int set, int stage, int kk) __attribute__((always_inline)) {
     const unsigned base = lds0 + unsigned(stage * STG), col = unsigned(((2 * kk + fc) ^ swz) << 4);
@@ -238,7 +300,7 @@ __global__ __launch_bounds__(WO * WP * 64) void nhwc_kernel(const uint16_t* __re
 #pragma unroll
     for (int i = 0; i < FP; ++i)
 #pragma unroll
-      for (int j = 0; j < FO; ++j) acc[i][j] = E::mfma32(af[set][i], bf[set][j], acc[i][j]);
+      for (int j = 0; j < FO; ++j) E::mma(af[set][i], bf[set][j], sum[i][j]);
   };
   wait_vmcnt<(NST - 1) * NI>();
   stage_barrier();
@@ -261,14 +323,34 @@ __global__ __launch_bounds__(WO * WP * 64) void nhwc_kernel(const uint16_t* __re
       __builtin_amdgcn_sched_barrier(0);
     }
     st = nx;
+    if (NA > 1 && (t - t_beg) % 16 == 15) add_up();
   }
   wait_vmcnt<0>();  // loads past the last step still target the stages
   __syncthreads();
-  if (g.split == 1) {
-    tile_to_y<E, TO, TP, WO, WP>(acc, lds, bias, y, tid, o0, n0, g.O, g.OHW, g.N, g.relu);
+  add_up();
+  float* part = partial + static_cast<long long>(z) * g.total;
+  const bool last = g.split == 1;
+  if constexpr (E::kDtype == GIE_HIP_FP32) {
+    if (last) {
+      part = static_cast<float*>(y);
+#pragma unroll
+      for (int j = 0; j < FO; ++j) {
+        const int o = o0 + wo * WTO + j * 32 + fr;
+        const float bv = bias != nullptr && o < g.O ? static_cast<const float*>(bias)[o] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < FP; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            acc[i][j][e] += bv;
+            if (g.relu) acc[i][j][e] = fmaxf(acc[i][j][e], 0.0f);
+          }
+      }
+    }
+  } else if (last) {
+    tile_to_y<E, TO, TP, WO, WP>(acc, lds, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), tid, o0, n0, g.O,
+                                 g.OHW, g.N, g.relu);
     return;
   }
-  float* part = partial + static_cast<long long>(z) * g.total;
 #pragma unroll
   for (int i = 0; i < FP; ++i) {
 #pragma unroll
@@ -301,13 +383,15 @@ __global__ __launch_bounds__(WO * WP * 64) void nhwc_kernel(const uint16_t* __re
 // ---- configurations: filters x pixels of the tile, threads, stages ----
 struct NhwcConfig {
   int to, tp, threads, stages;
+  bool f32;  // four accumulators fit the registers two workgroups share
 };
 constexpr NhwcConfig kNhwcConfigs[] = {
-    {64, 64, 256, 4}, {64, 128, 256, 3}, {128, 128, 512, 3}, {128, 256, 512, 3}, {256, 256, 512, 2},
+    {64, 64, 256, 4, true},    {64, 128, 256, 3, false},  {128, 128, 512, 3, true},
+    {128, 256, 512, 3, false}, {256, 256, 512, 2, false},
 };
 constexpr int kNhwcCount = int(sizeof(kNhwcConfigs) / sizeof(kNhwcConfigs[0]));
 
-using NhwcFn = void (*)(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, float*, NhwcGeom);
+using NhwcFn = void (*)(const uint16_t*, const uint16_t*, const void*, void*, float*, NhwcGeom);
 
 template <typename E>
 NhwcFn nhwc_fn(int config) {
@@ -320,14 +404,21 @@ NhwcFn nhwc_fn(int config) {
   }
 }
 
-int nhwc_prepare(int config, const gie_conv_geom* gg, int split, NhwcGeom* g, int* lds, long long* blocks) {
+NhwcFn nhwc_fn32(int config) {
+  return config == 0 ? &nhwc_kernel<NhF32, 64, 64, 2, 2, 4> : &nhwc_kernel<NhF32, 128, 128, 2, 4, 3>;
+}
+
+int nhwc_prepare(int config, int dtype, const gie_conv_geom* gg, int split, NhwcGeom* g, int* lds, long long* blocks) {
   if (!gg || config < 0 || config >= kNhwcCount || split < 1 || split > 64) return GIE_HIP_EINVAL;
+  if (dtype != GIE_HIP_FP16 && dtype != GIE_HIP_BF16 && (dtype != GIE_HIP_FP32 || !kNhwcConfigs[config].f32))
+    return GIE_HIP_EUNSUPPORTED;
+  const int unit = dtype == GIE_HIP_FP32 ? 2 : 1;  // 16-bit units of an element
   if (gg->batch <= 0 || gg->in_channels <= 0 || gg->in_h <= 0 || gg->in_w <= 0 || gg->out_channels <= 0 ||
       gg->kernel_h <= 0 || gg->kernel_w <= 0 || gg->stride_h <= 0 || gg->stride_w <= 0 || gg->pad_h < 0 ||
       gg->pad_w < 0 || gg->out_h <= 0 || gg->out_w <= 0)
     return GIE_HIP_EINVAL;
   const NhwcConfig& nc = kNhwcConfigs[config];
-  const long long cp = (gg->in_channels + 7) / 8 * 8, hp = gg->in_h + 2LL * gg->pad_h, wp = gg->in_w + 2LL * gg->pad_w;
+  const long long cp = (1LL * gg->in_channels * unit + 7) / 8 * 8, hp = gg->in_h + 2LL * gg->pad_h, wp = gg->in_w + 2LL * gg->pad_w;
   if ((gg->out_h - 1LL) * gg->stride_h + gg->kernel_h > hp || (gg->out_w - 1LL) * gg->stride_w + gg->kernel_w > wp)
     return GIE_HIP_EINVAL;
   const long long run = gg->kernel_w * cp, steps = (run + 63) / 64, kp = steps * 64 * gg->kernel_h;
@@ -337,7 +428,7 @@ int nhwc_prepare(int config, const gie_conv_geom* gg, int split, NhwcGeom* g, in
     return GIE_HIP_EUNSUPPORTED;
   const long long t = steps * gg->kernel_h;
   if (t < split) return GIE_HIP_EUNSUPPORTED;
-  *lds = std::max(nc.stages * (nc.to + nc.tp) * 128, nc.to * (nc.tp * 2 + 16));
+  *lds = std::max(nc.stages * (nc.to + nc.tp) * 128, unit == 1 ? nc.to * (nc.tp * 2 + 16) : 0);
   const long long n_pt = (n + nc.tp - 1) / nc.tp, n_ot = (gg->out_channels + nc.to - 1) / nc.to;
   *blocks = (n_pt + 7) / 8 * 8 * n_ot * split;
   if (*blocks > 0x7fffffffLL) return GIE_HIP_EUNSUPPORTED;
@@ -356,6 +447,27 @@ int nhwc_prepare(int config, const gie_conv_geom* gg, int split, NhwcGeom* g, in
 
 bool off_by(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; }
 
+template <typename T>
+int repack_nhwc(const NhwcGeom& g, int batch, const void* x, void* xp, const void* w, void* wp, void* stream) {
+  constexpr int unit = int(sizeof(T)) / 2;
+  NhwcRepack<T> j;
+  j.x = static_cast<const T*>(x), j.w = static_cast<const T*>(w);
+  j.xp = static_cast<T*>(xp), j.wp = static_cast<T*>(wp);
+  j.B = batch, j.C = g.C, j.H = g.H, j.W = g.W, j.HW = g.H * g.W, j.Cp = g.Cp / unit, j.Hp = g.Hp, j.Wp = g.Wp;
+  j.PH = g.PH, j.PW = g.PW, j.O = g.O, j.KH = g.KH, j.KW = g.KW, j.Kp = g.Kp / unit, j.run = g.run_steps * 64 / unit;
+  j.gpi = ((j.HW + 3) / 4 + 15) / 16 * 16;
+  j.cgs = (g.Cp + 31) / 32;
+  j.x_waves = 1LL * batch * (j.gpi / 16) * j.cgs;
+  j.x_blocks = (j.x_waves + 3) / 4;
+  j.border = 1LL * batch * (1LL * g.Hp * g.Wp - j.HW) * (g.Cp / 8);
+  j.b_blocks = (j.border + kNhThreads - 1) / kNhThreads;
+  const long long total = j.x_blocks + j.b_blocks + g.O;
+  if (total > 0x7fffffffLL) return GIE_HIP_EUNSUPPORTED;
+  hipLaunchKernelGGL(nhwc_repack_kernel<T>, dim3(unsigned(total)), dim3(kNhThreads), 0, static_cast<hipStream_t>(stream), j);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? GIE_HIP_OK : int(e);
+}
+
 }  // namespace
 }  // namespace gie_hip
 
@@ -371,12 +483,12 @@ extern "C" int gie_hip_nhwc_config_get(int config, int* tile_m, int* tile_n, int
   return GIE_HIP_OK;
 }
 
-extern "C" int gie_hip_nhwc_check(int config, const gie_conv_geom* gg, long long* x_bytes, long long* w_bytes, int* steps,
-                                  int* lds_bytes) {
+extern "C" int gie_hip_nhwc_check(int config, int dtype, const gie_conv_geom* gg, long long* x_bytes, long long* w_bytes,
+                                  int* steps, int* lds_bytes) {
   NhwcGeom g;
   int lds = 0;
   long long blocks = 0;
-  const int rc = nhwc_prepare(config, gg, 1, &g, &lds, &blocks);
+  const int rc = nhwc_prepare(config, dtype, gg, 1, &g, &lds, &blocks);
   if (rc != GIE_HIP_OK) return rc;
   if (x_bytes) *x_bytes = g.xp_bytes;
   if (w_bytes) *w_bytes = g.wp_bytes;
@@ -385,45 +497,35 @@ extern "C" int gie_hip_nhwc_check(int config, const gie_conv_geom* gg, long long
   return GIE_HIP_OK;
 }
 
-extern "C" int gie_hip_repack_nhwc(const void* x, void* xp, const void* w, void* wp, const gie_conv_geom* gg, void* stream) {
+extern "C" int gie_hip_repack_nhwc(int dtype, const void* x, void* xp, const void* w, void* wp, const gie_conv_geom* gg,
+                                   void* stream) {
   if (!x || !xp || !w || !wp) return GIE_HIP_EINVAL;
   NhwcGeom g;
   int lds = 0;
   long long blocks = 0;
-  if (int rc = nhwc_prepare(0, gg, 1, &g, &lds, &blocks)) return rc;
-  if (off_by(x, 2) || off_by(w, 2) || off_by(xp, 16) || off_by(wp, 16)) return GIE_HIP_EINVAL;
-  NhwcRepack j;
-  j.x = static_cast<const uint16_t*>(x), j.w = static_cast<const uint16_t*>(w);
-  j.xp = static_cast<uint16_t*>(xp), j.wp = static_cast<uint16_t*>(wp);
-  j.B = gg->batch, j.C = g.C, j.H = g.H, j.W = g.W, j.HW = g.H * g.W, j.Cp = g.Cp, j.Hp = g.Hp, j.Wp = g.Wp;
-  j.PH = g.PH, j.PW = g.PW, j.O = g.O, j.KH = g.KH, j.KW = g.KW, j.Kp = g.Kp, j.run = g.run_steps * 64;
-  j.gpi = ((j.HW + 3) / 4 + 15) / 16 * 16;
-  j.cgs = (g.Cp + 31) / 32;
-  j.x_waves = 1LL * gg->batch * (j.gpi / 16) * j.cgs;
-  j.x_blocks = (j.x_waves + 3) / 4;
-  j.border = 1LL * gg->batch * (1LL * g.Hp * g.Wp - j.HW) * (g.Cp / 8);
-  j.b_blocks = (j.border + kNhThreads - 1) / kNhThreads;
-  const long long total = j.x_blocks + j.b_blocks + g.O;
-  if (total > 0x7fffffffLL) return GIE_HIP_EUNSUPPORTED;
-  hipLaunchKernelGGL(nhwc_repack_kernel, dim3(unsigned(total)), dim3(kNhThreads), 0, static_cast<hipStream_t>(stream), j);
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? GIE_HIP_OK : int(e);
+  if (int rc = nhwc_prepare(0, dtype, gg, 1, &g, &lds, &blocks)) return rc;
+  const uintptr_t es = dtype == GIE_HIP_FP32 ? 4 : 2;
+  if (off_by(x, es) || off_by(w, es) || off_by(xp, 16) || off_by(wp, 16)) return GIE_HIP_EINVAL;
+  return dtype == GIE_HIP_FP32 ? repack_nhwc<uint32_t>(g, gg->batch, x, xp, w, wp, stream)
+                               : repack_nhwc<uint16_t>(g, gg->batch, x, xp, w, wp, stream);
 }
 
 extern "C" int gie_hip_conv_nhwc(int config, int dtype, const gie_conv_geom* gg, const void* xp, const void* wp,
                                  const void* bias, void* y, float* partial, int split, void* stream) {
   if (!xp || !wp || (split == 1 && !y) || (split > 1 && !partial)) return GIE_HIP_EINVAL;
-  if (dtype != GIE_HIP_FP16 && dtype != GIE_HIP_BF16) return GIE_HIP_EUNSUPPORTED;
   NhwcGeom g;
   int lds = 0;
   long long blocks = 0;
-  if (int rc = nhwc_prepare(config, gg, split, &g, &lds, &blocks)) return rc;
-  if (off_by(xp, 16) || off_by(wp, 16) || off_by(y, 2) || off_by(bias, 2) || off_by(partial, 4)) return GIE_HIP_EINVAL;
-  const NhwcFn fn = dtype == GIE_HIP_FP16 ? nhwc_fn<Fp16>(config) : nhwc_fn<Bf16>(config);
+  if (int rc = nhwc_prepare(config, dtype, gg, split, &g, &lds, &blocks)) return rc;
+  const uintptr_t es = dtype == GIE_HIP_FP32 ? 4 : 2;
+  if (off_by(xp, 16) || off_by(wp, 16) || off_by(y, es) || off_by(bias, es) || off_by(partial, 4)) return GIE_HIP_EINVAL;
+  const NhwcFn fn = dtype == GIE_HIP_FP16   ? nhwc_fn<NhHalf<Fp16>>(config)
+                    : dtype == GIE_HIP_BF16 ? nhwc_fn<NhHalf<Bf16>>(config)
+                                            : nhwc_fn32(config);
   if (int rc = set_lds_limit(reinterpret_cast<const void*>(fn), lds)) return rc;
   hipLaunchKernelGGL(fn, dim3(unsigned(blocks)), dim3(unsigned(kNhwcConfigs[config].threads)), size_t(lds),
                      static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(xp), static_cast<const uint16_t*>(wp),
-                     static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), partial, g);
+                     bias, y, partial, g);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? GIE_HIP_OK : int(e);
 }

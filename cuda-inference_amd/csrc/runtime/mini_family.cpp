@@ -84,7 +84,8 @@ double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   // weights element by element (3x3, 331 channels: 44 us)
   if (k16 && p.gemm_k() % 2 != 0) per_load *= one || nine ? 3.5 : 1.4;
   // strided rows of x take twice the cache lines (1x1 544 -> 32, 29x29 /2, batch 53: 37 us at 16x16)
-  if (k16 && (one || nine) && p.stride_w > 1 && wave > 1.0) per_load *= 1.6;
+  // FP32: 1x1 466 -> 384, 22x22 /2, batch 60: 85 us, twice the unstrided rate's
+  if ((one || (k16 && nine)) && p.stride_w > 1 && wave > 1.0) per_load *= k16 ? 1.6 : 2.0;
   const double share = k16 ? 0.5 * (wave + std::ceil(wave)) : wave;  // the last wave of workgroups is partly empty
   // a CU with a single workgroup is bound by its latency, not by its load path (1024 -> 256, 196 pixels: 5.7 us)
   if (k16 && one && t == 32) per_load -= 0.0038 * std::max(0.0, 2.0 - share);

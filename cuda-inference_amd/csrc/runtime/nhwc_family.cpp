@@ -8,11 +8,13 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <string>
 #include <vector>
 
 #include "gie_hip.h"
 #include "gpu_inference/kernel_registry.h"
+#include "nhwc_family.h"
 
 namespace gie {
 namespace {
@@ -40,7 +42,9 @@ gie_conv_geom geom_of(const ConvProblem& prob) {
   return g;
 }
 
-int dtype_of(Precision p) { return p == Precision::kFp16 ? GIE_HIP_FP16 : GIE_HIP_BF16; }
+int dtype_of(Precision p) {
+  return p == Precision::kFp16 ? GIE_HIP_FP16 : p == Precision::kBf16 ? GIE_HIP_BF16 : GIE_HIP_FP32;
+}
 
 struct Tile {
   int m = 1, n = 1, threads = 64;
@@ -60,9 +64,33 @@ Plan plan_of(int config, const ConvProblem& prob) {
   const gie_conv_geom g = geom_of(prob);
   long long xb = 0, wb = 0;
   Plan p;
-  p.ok = gie_hip_nhwc_check(config, &g, &xb, &wb, &p.steps, &p.lds) == GIE_HIP_OK;
+  p.ok = gie_hip_nhwc_check(config, dtype_of(prob.precision), &g, &xb, &wb, &p.steps, &p.lds) == GIE_HIP_OK;
   p.x_bytes = size_t(xb), p.w_bytes = size_t(wb);
   return p;
+}
+
+// One call: repack, GEMM, reduce where split; `ws` holds [x | w | partials], each 256-byte aligned.
+void run(int config, int split, const LaunchArgs& la) {
+  const ConvProblem& prob = *la.problem;
+  const gie_conv_geom g = geom_of(prob);
+  const Plan pl = plan_of(config, prob);
+  char* ws = static_cast<char*>(la.workspace);
+  void* wp = ws + align256(pl.x_bytes);
+  float* part = split > 1 ? reinterpret_cast<float*>(ws + align256(pl.x_bytes) + align256(pl.w_bytes)) : nullptr;
+  const int dt = dtype_of(prob.precision);
+  const auto stage = [&](int k) { return la.only_stage < 0 || la.only_stage == k; };
+  record_stage_event(la, 0);
+  if (stage(0))
+    check_kernel_status(gie_hip_repack_nhwc(dt, la.x, ws, la.w, wp, &g, la.stream), "repack (padded NHWC, filter runs)");
+  record_stage_event(la, 1);
+  if (stage(1))
+    check_kernel_status(gie_hip_conv_nhwc(config, dt, &g, ws, wp, la.bias, la.y, part, split, la.stream),
+                        "padded-NHWC MFMA convolution");
+  record_stage_event(la, 2);
+  if (split > 1 && stage(2))
+    check_kernel_status(gie_hip_splitk_reduce(dt, part, la.bias, la.y, prob.p.output_shape().numel(), split,
+                                              prob.p.out_channels, g.out_h * g.out_w, g.relu, la.stream),
+                        "split-K reduce");
 }
 
 template <int Config, int Split, Precision P>
@@ -113,28 +141,7 @@ struct Fns {
     return f.fixed + moved / 4.3e6 + reduce +
            std::max(f.alone + steps * f.alone_step, share * (f.start + steps * f.step));
   }
-  static void launch(const LaunchArgs& la) {
-    const ConvProblem& prob = *la.problem;
-    const gie_conv_geom g = geom_of(prob);
-    const Plan pl = plan_of(Config, prob);
-    char* ws = static_cast<char*>(la.workspace);
-    void* wp = ws + align256(pl.x_bytes);
-    float* part = Split > 1 ? reinterpret_cast<float*>(ws + align256(pl.x_bytes) + align256(pl.w_bytes)) : nullptr;
-    const int dt = dtype_of(P);
-    const auto stage = [&](int k) { return la.only_stage < 0 || la.only_stage == k; };
-    record_stage_event(la, 0);
-    if (stage(0))
-      check_kernel_status(gie_hip_repack_nhwc(la.x, ws, la.w, wp, &g, la.stream), "repack (padded NHWC, filter runs)");
-    record_stage_event(la, 1);
-    if (stage(1))
-      check_kernel_status(gie_hip_conv_nhwc(Config, dt, &g, ws, wp, la.bias, la.y, part, Split, la.stream),
-                          "padded-NHWC MFMA convolution");
-    record_stage_event(la, 2);
-    if (Split > 1 && stage(2))
-      check_kernel_status(gie_hip_splitk_reduce(dt, part, la.bias, la.y, prob.p.output_shape().numel(), Split,
-                                                prob.p.out_channels, g.out_h * g.out_w, g.relu, la.stream),
-                          "split-K reduce");
-  }
+  static void launch(const LaunchArgs& la) { run(Config, Split, la); }
 };
 
 template <int Config, int Split, Precision P>
@@ -178,6 +185,37 @@ void add_precision(std::vector<KernelDesc>& out) {
 }
 
 }  // namespace
+
+// Per tile: fixed cost, the repack at its traffic, each CU's whole share of the workgroups at a start-up cost and a cost for
+// each 32-channel step, the reduce. Fitted to 75 layers on one MI355X (4-7 % rms).
+NhwcF32 nhwc_f32_best(const ConvProblem& prob, int cus, size_t room) {
+  struct Fit {
+    int config;
+    double fixed, alone_step, start, step;
+  };
+  constexpr Fit kFit[] = {{0, 5.2, 0.617, 0.8, 0.526}, {2, 4.5, 1.945, 2.95, 1.945}};
+  NhwcF32 best;
+  for (const Fit& f : kFit) {
+    const Plan pl = plan_of(f.config, prob);
+    if (!pl.ok) continue;
+    const Tile t = tile_of(f.config);
+    const double y = double(prob.p.output_shape().numel()) * 4;
+    const double moved = double(pl.x_bytes) + double(prob.p.input_shape().numel()) * 4 + 2.0 * double(pl.w_bytes);
+    const int64_t tiles = (prob.p.gemm_n() + t.n - 1) / t.n * ((prob.p.out_channels + t.m - 1) / t.m);
+    for (int split : {1, 2, 4}) {
+      if (split > 1 && pl.steps < 4 * split) continue;
+      const size_t part = split > 1 ? align256(size_t(split) * size_t(y)) : 0;
+      if (align256(pl.x_bytes) + align256(pl.w_bytes) + part > room) continue;
+      const double share = std::ceil(double(tiles * split) / std::max(cus, 1)), steps = double(pl.steps) / split;
+      const double us = f.fixed + moved / 4.3e6 + std::max(steps * f.alone_step, share * (f.start + steps * f.step)) +
+                        (split > 1 ? 1.5 + 0.27 * (split + 1) * y / 1e6 : 0.0);
+      if (best.config < 0 || us < best.us) best.config = f.config, best.split = split, best.us = us;
+    }
+  }
+  return best;
+}
+
+void nhwc_f32_launch(const NhwcF32& how, const LaunchArgs& la) { run(how.config, how.split, la); }
 
 void register_nhwc_family(std::vector<KernelDesc>& out) {
   if (gie_hip_nhwc_config_count() != 5) throw Error(StatusCode::kInternal, "padded-NHWC tile table changed");

@@ -222,8 +222,8 @@ _HIP = {
     "gie_hip_conv_gather": ([_i, _i, _GP, _vp, _vp, _vp, _vp, _vp], _i),
     "gie_hip_nhwc_config_count": ([], _i),
     "gie_hip_nhwc_config_get": ([_i, _ip, _ip, _ip], _i),
-    "gie_hip_nhwc_check": ([_i, _GP, ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(ctypes.c_longlong), _ip, _ip], _i),
-    "gie_hip_repack_nhwc": ([_vp, _vp, _vp, _vp, _GP, _vp], _i),
+    "gie_hip_nhwc_check": ([_i, _i, _GP, ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(ctypes.c_longlong), _ip, _ip], _i),
+    "gie_hip_repack_nhwc": ([_i, _vp, _vp, _vp, _vp, _GP, _vp], _i),
     "gie_hip_conv_nhwc": ([_i, _i, _GP, _vp, _vp, _vp, _vp, _vp, _i, _vp], _i),
     "gie_hip_slab_config_count": ([], _i),
     "gie_hip_slab_config_get": ([_i, ctypes.POINTER(GieSlabConfig)], _i),

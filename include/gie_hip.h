@@ -253,16 +253,19 @@ int gie_hip_conv_gather(int config, int dtype, const gie_conv_geom* g, const voi
                         void* y, void* stream);
 
 /* Convolution of any filter, stride and padding over a spatially padded NHWC copy of x (two launches):
-   gie_hip_repack_nhwc fills xp (x_bytes of _check: [batch][in_h + 2 pad_h][in_w + 2 pad_w][channels rounded up to 8], the
-   padding as zeros) and wp (w_bytes: [out_channels][kernel_h][run], run = kernel_w * padded channels rounded up to 64),
+   gie_hip_repack_nhwc fills xp (x_bytes of _check: [batch][in_h + 2 pad_h][in_w + 2 pad_w][channels rounded up to 16
+   bytes], the padding as zeros) and wp (w_bytes: [out_channels][kernel_h][run], run = kernel_w * padded channels rounded
+   up to 128 bytes),
    both 16-byte aligned; gie_hip_conv_nhwc multiplies them: fused bias + ReLU into y for split 1, FP32 partials
    partial[split][NCHW] for split > 1 (at most the `steps` of _check; reduce with gie_hip_splitk_reduce). dtype
-   GIE_HIP_FP16 / _BF16; x, w, y and bias 2-byte aligned. _config_get: filters x pixels per workgroup and its threads. */
+   GIE_HIP_FP16 / _BF16, or GIE_HIP_FP32 for the configurations _check accepts it for (in_channels then in FP32
+   elements, FP32 sums over quarters of the reduction); x, w, y and bias aligned to their element. _config_get: filters x pixels per workgroup and its threads. */
 int gie_hip_nhwc_config_count(void);
 int gie_hip_nhwc_config_get(int config, int* tile_m, int* tile_n, int* threads);
-int gie_hip_nhwc_check(int config, const gie_conv_geom* g, long long* x_bytes, long long* w_bytes, int* steps,
+int gie_hip_nhwc_check(int config, int dtype, const gie_conv_geom* g, long long* x_bytes, long long* w_bytes, int* steps,
                        int* lds_bytes);
-int gie_hip_repack_nhwc(const void* x, void* xp, const void* w, void* wp, const gie_conv_geom* g, void* stream);
+int gie_hip_repack_nhwc(int dtype, const void* x, void* xp, const void* w, void* wp, const gie_conv_geom* g,
+                        void* stream);
 int gie_hip_conv_nhwc(int config, int dtype, const gie_conv_geom* g, const void* xp, const void* wp, const void* bias,
                       void* y, float* partial, int split, void* stream);
 

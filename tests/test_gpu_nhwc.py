@@ -48,7 +48,7 @@ def test_nhwc_repack_is_bit_exact(case):
     w = rng.integers(0, 1 << 16, p.w_shape(), dtype=np.uint16)
     g = p.geom(C)
     xb, wb = ctypes.c_longlong(), ctypes.c_longlong()
-    assert gie.hip().gie_hip_nhwc_check(0, ctypes.byref(g), ctypes.byref(xb), ctypes.byref(wb), None, None) == 0
+    assert gie.hip().gie_hip_nhwc_check(0, 1, ctypes.byref(g), ctypes.byref(xb), ctypes.byref(wb), None, None) == 0
     cp = (C + 7) // 8 * 8
     run = (KW * cp + 63) // 64 * 64
     assert xb.value == 2 * B * (H + 2 * PH) * (W + 2 * PW) * cp and wb.value == 2 * Oc * KH * run
@@ -59,7 +59,7 @@ def test_nhwc_repack_is_bit_exact(case):
         xp, wp = gie.DeviceBuffer(xb.value), gie.DeviceBuffer(wb.value)
         xp.fill(0xFF)
         wp.fill(0xFF)
-        gie.check_hip(gie.hip().gie_hip_repack_nhwc(dx.addr + off, xp.addr, dw.addr + off, wp.addr, ctypes.byref(g), None),
+        gie.check_hip(gie.hip().gie_hip_repack_nhwc(1, dx.addr + off, xp.addr, dw.addr + off, wp.addr, ctypes.byref(g), None),
                       "repack")
         gie.synchronize()
         want = np.zeros((B, H + 2 * PH, W + 2 * PW, cp), np.uint16)
@@ -106,15 +106,63 @@ def test_nhwc_pads_a_run_with_zeros_on_both_sides():
     assert np.array_equal(t.y()[:, :, :, :7], ref[:, :, :, :7])
 
 
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_nhwc_fp32(case):
+    """Both FP32 tiles and a split through the C-ABI, every tensor one element into its allocation."""
+    p = _problem(case, "fp32")
+    b = Bundle(p, 0x3F + CASES.index(case), O.NORMAL)
+    g, h, n = p.geom(p.in_channels), gie.hip(), int(np.prod(p.y_shape()))
+    dx, dw, db, y = (gie.DeviceBuffer(v + 16) for v in (b.x.nbytes, b.w.nbytes, 4 * p.out_channels, 4 * n))
+    dx.upload(b.x.astype(np.float32), 4)
+    dw.upload(b.w.astype(np.float32), 4)
+    if b.b is not None:
+        db.upload(b.b.astype(np.float32), 4)
+    bias = db.addr + 4 if p.has_bias else None
+    for config in (0, 2):
+        xb, wb, steps = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
+        assert h.gie_hip_nhwc_check(config, 0, ctypes.byref(g), ctypes.byref(xb), ctypes.byref(wb), ctypes.byref(steps),
+                                    None) == 0
+        xp, wp, part = gie.DeviceBuffer(xb.value), gie.DeviceBuffer(wb.value), gie.DeviceBuffer(8 * n)
+        for split in (1, 2):
+            if steps.value < split:
+                continue
+            for d in (xp, wp, part, y):
+                d.fill(0xFF)
+            gie.check_hip(h.gie_hip_repack_nhwc(0, dx.addr + 4, xp.addr, dw.addr + 4, wp.addr, ctypes.byref(g), None), "r")
+            gie.check_hip(h.gie_hip_conv_nhwc(config, 0, ctypes.byref(g), xp.addr, wp.addr, bias, y.addr + 4,
+                                              part.addr if split > 1 else None, split, None), "conv")
+            if split > 1:
+                gie.check_hip(h.gie_hip_splitk_reduce(0, part.addr, bias, y.addr + 4, n, split, p.out_channels,
+                                                      p.out_h * p.out_w, int(p.relu), None), "reduce")
+            gie.synchronize()
+            m = b.compare(y.download(np.float32, n + 1)[1:].reshape(p.y_shape()))
+            assert m.passed(), f"config {config} split {split}: {m.summary()}"
+
+
+@pytest.mark.parametrize("case", [(32, 128, 28, 28, 128, 3, 3, 1, 1, 1), (8, 3, 112, 112, 64, 7, 7, 2, 3, 3),
+                                  (2, 24, 9, 9, 32, 3, 3, 1, 1, 1)], ids=lambda c: "x".join(map(str, c)))
+def test_nhwc_fp32_through_the_split_8_entry(case):
+    """The FP32 entry that runs these kernels where they are faster: its workspace is its own eight partials."""
+    name = "implicit_gemm_fp32_128x128x16_mfma_sk8"
+    p = gie.Problem(*case[:8], case[7], *case[8:], precision="fp32", has_bias=True, relu=True)
+    b = Bundle(p, 0x8E, O.NORMAL, full_reference=False, sample=4096)
+    assert gie.Plan(p, name).workspace_bytes == (8 * 4 * int(np.prod(p.y_shape())) + 255) // 256 * 256
+    y, why = run_plan(name, b, repeats=2)
+    assert y is not None, why
+    m = b.compare(y)
+    assert m.passed(), m.summary()
+
+
 def test_nhwc_argument_checks():
     h = gie.hip()
     ok = gie.Problem(1, 16, 5, 5, 16, 3, 3, 1, 1, 1, 1, precision="fp16")
     g, d = ok.geom(16), gie.DeviceBuffer(1 << 20)
-    assert h.gie_hip_nhwc_check(h.gie_hip_nhwc_config_count(), ctypes.byref(g), None, None, None, None) == -1
+    assert h.gie_hip_nhwc_check(h.gie_hip_nhwc_config_count(), 1, ctypes.byref(g), None, None, None, None) == -1
     far = gie.Problem(64, 1024, 224, 224, 16, 3, 3, 1, 1, 1, 1, precision="fp16")
-    assert h.gie_hip_nhwc_check(0, ctypes.byref(far.geom(1024)), None, None, None, None) == -2
-    assert h.gie_hip_conv_nhwc(0, 0, ctypes.byref(g), d.addr, d.addr, None, d.addr, None, 1, None) == -2   # fp32
+    assert h.gie_hip_nhwc_check(0, 1, ctypes.byref(far.geom(1024)), None, None, None, None) == -2
+    assert h.gie_hip_conv_nhwc(0, 3, ctypes.byref(g), d.addr, d.addr, None, d.addr, None, 1, None) == -2   # tf32
+    assert h.gie_hip_nhwc_check(1, 0, ctypes.byref(g), None, None, None, None) == -2  # fp32: 64x64 and 128x128 only
     assert h.gie_hip_conv_nhwc(0, 1, ctypes.byref(g), d.addr + 8, d.addr, None, d.addr, None, 1, None) == -1
     assert h.gie_hip_conv_nhwc(0, 1, ctypes.byref(g), d.addr, d.addr, None, d.addr, None, 2, None) == -1   # no partials
     assert h.gie_hip_conv_nhwc(0, 1, ctypes.byref(g), d.addr, d.addr, None, d.addr, d.addr, 4, None) == -2  # 3 steps
-    assert h.gie_hip_repack_nhwc(d.addr + 1, d.addr, d.addr, d.addr, ctypes.byref(g), None) == -1
+    assert h.gie_hip_repack_nhwc(1, d.addr + 1, d.addr, d.addr, d.addr, ctypes.byref(g), None) == -1

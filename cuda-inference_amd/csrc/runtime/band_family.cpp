@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <string>
 #include <vector>
 
@@ -153,7 +154,8 @@ struct Fns {
     const Entry& en = e();
     const bool wide = en.info.tile_n == 256;
     const double slices = double(slices_of(prob, en)) / en.split;
-    const double share = double(blocks(prob)) / std::max(cus, 1);
+    const double rounds = double(blocks(prob)) / std::max(cus, 1);
+    const double share = 0.5 * (rounds + std::ceil(rounds));  // the last round is partly empty
     const double y = double(prob.p.output_shape().numel()) / 1e6;  // million outputs
     const double wp = double(prob.p.out_channels) * prob.p.kernel_h * prob.p.kernel_w * c_pad_of(prob) * 2.0 / 1e6;
     const double reduce = en.split > 1 ? (en.split + 1) * 4.0 * y * (wide ? 0.47 : 0.26) : 0.0;

@@ -77,7 +77,7 @@ double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   // operand loads of a lane over the reduction's whole supersteps (3x3: 9 chunks of each lane group, else 64 k)
   const int64_t ss = nine ? 9 * (64 / t) * ck : 8 * ck;
   const double loads = double((p.gemm_k() + ss - 1) / ss * ss) / (ck * (64 / t)) * (ck + 1);
-  double per_load = !one && !nine ? (t == 16 ? 0.014 : 0.022) : !k16 ? 0.012 : t == 16 && one ? 0.0057 : 0.0085;
+  double per_load = !one && !nine ? (t == 16 ? 0.014 : k16 ? 0.0105 : 0.022) : !k16 ? 0.012 : t == 16 && one ? 0.0057 : 0.0085;
   const double wave = std::max(1.0, double(blocks_of(config, prob)) / std::max(cus, 1));
   if (waves_of(config) == 16 && (one || nine || wave <= 1.0))
     per_load *= !one && !nine ? 0.85 : k16 ? 1.0 : one ? 0.7 : 0.95;
@@ -89,7 +89,11 @@ double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   const double share = k16 ? 0.5 * (wave + std::ceil(wave)) : wave;  // the last wave of workgroups is partly empty
   // a CU with a single workgroup is bound by its latency, not by its load path (1024 -> 256, 196 pixels: 5.7 us)
   if (k16 && one && t == 32) per_load -= 0.0038 * std::max(0.0, 2.0 - share);
-  const double start = t != 16 ? 1.0 : k16 && one ? 0.7 : 1.3;
+  // filters without an unrolled form set up their taps for each workgroup, which a CU with one hides in part (1x3 32 ->
+  // 143 over 43x43: 15 us); 3x3 workgroups beyond two a CU queue on the load path
+  double start = t != 16 ? 1.0 : k16 && one ? 0.7 : 1.3;
+  if (k16 && t == 32 && !one && !nine) start = wave > 1.0 ? 3.6 : 2.2;
+  if (k16 && t == 32 && nine && wave > 2.0) start *= 1.3, per_load *= 1.15;
   return 0.5 + share * (start + loads * per_load) + (t == 16 ? 0.7 * (share - 1.0) : 0.0);
 }
 

@@ -80,11 +80,12 @@ int full_form_of(const Entry& en) {
 
 // Steady-state rate of each form against the split form's, whose profile the family carries (MI355X, FP16 3x3 256 -> 256
 // over 14x14, batch 32 / 288 -> 367 over 12x12, batch 22: split 9.1 / 15.6 us, pipelined 10.3 / 17.7, two lean
-// workgroups a CU 15.1 / 19.8, full 16.0 / 28.8). Taking them for equal made the dispatcher choose the full form.
+// workgroups a CU 15.1 / 19.8, full 16.0 / 28.8; the full form of the 4- and 8-row slabs is nearer). Taking them for equal made the dispatcher choose the full form.
 double rate_of(const gie_slab_config& info) {
   if (info.form == 3) return 1.0;
   if (info.form == 2) return 0.82;
-  return info.workgroups_per_cu > 1 ? 0.95 : 0.46;
+  if (info.workgroups_per_cu > 1) return 0.95;
+  return info.form == 0 && info.rows < 14 ? 0.6 : 0.46;
 }
 
 template <int I>

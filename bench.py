@@ -299,6 +299,9 @@ def dominant_kernel(registry_name: str) -> str:
              ("stem_", "stem_kernel (7x7 stride-2 stem straight from NCHW, conv_stem.hip)"),
              ("narrow_", "narrow_kernel (3x3, whole reduction per workgroup, conv_narrow.hip)"),
              ("stack_", "stack_kernel (3x3 MFMA convolution of small images stacked per workgroup, conv_stack.hip)"),
+             ("mini_", "mini_kernel (small MFMA convolutions straight from NCHW / OIHW, conv_mini.hip)"),
+             ("gather_", "gather_kernel (1x1 MFMA convolution of any stride straight from NCHW, conv_gather.hip)"),
+             ("nhwc_", "nhwc_kernel (padded-NHWC MFMA implicit GEMM, conv_nhwc.hip)"),
              ("implicit_gemm_fp32_", "f32_kernel (FP32 MFMA convolution, conv_f32.hip)"),
              ("mfma_tf32_", "f32_kernel (TF32 MFMA convolution, conv_f32.hip)")]
     for stem, fn in stems:

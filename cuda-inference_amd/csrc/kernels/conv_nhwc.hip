@@ -13,11 +13,11 @@
 //   * GEMM: TO filters x TP pixels per workgroup, NST stages of LDS rows [pixel or filter][64 k] filled by 16-byte
 //     direct-to-LDS loads (16-byte chunk c of row r in slot c ^ ((r >> 1) & 7): 16 rows of an operand read cover the 64
 //     banks; the permutation is in the lanes' source addresses), NST - 1 steps in flight, counted waits, one barrier
-//     per step, the next fragments read while the current ones multiply. Where a run is no multiple of 64, the lanes past its end load zeros in its last step (the weights there
-//     are zeros too, but x could be infinite);
+//     per step, the next fragments read while the current ones multiply. Where a run is no multiple of 64, the lanes past
+//     its end load zeros in its last step (the weights there are zeros too, but x could be infinite);
 // What bounds it now: LDS, at about 85 bytes per clock and CU for operand reads and direct loads together (neither more
 // stages, nor unpermuted loads, nor fragments read a step ahead change a step's time), hence the 256 x 256 tile for the
-// largest layers. Measured (both launches): BF16 3x3 256 -> 256 over 56x56, batch 16: 124 -> 81 us; FP16 3x3 64 -> 64 over
+// largest layers. Measured (both launches): BF16 3x3 256 -> 256 over 56x56, batch 16: 118.9 -> 71.8 us; FP16 3x3 64 -> 64 over
 // 56x56, batch 32: 33.8 -> 26 (best of the other kernels; 53 for the one the dispatcher took); 3x3 stride 2 128 -> 128
 // over 56x56, batch 32: 32.6 -> 26.
 //   * output through an LDS tile as whole rows (tile_epilogue.h), or FP32 partials for split-K (splitk_reduce.hip sums
@@ -36,7 +36,7 @@ namespace {
 // four are added into the tile's sums, so that no sum runs over more than 128 products and the error does not grow with
 // the reduction (3x3 512 channels: 1.4e-7 of the norm, 4.0e-7 for one chain). Here the matrix cores bound: a step runs at
 // 0.81 (64 x 64) and 0.88 (128 x 128) of their rate, the rest is the last round of tiles and the repack. Measured: 3x3
-// 128 -> 128 over 28x28, batch 32: 118 -> 92 us; 64 -> 64 over 56x56, batch 32: 148 -> 97; 7x7 stride 2 3 -> 64 over
+// 128 -> 128 over 28x28, batch 32: 118.7 -> 90.0 us; 64 -> 64 over 56x56, batch 32: 148 -> 97; 7x7 stride 2 3 -> 64 over
 // 224x224, batch 8: 119 -> 50.
 struct NhF32 {
   static constexpr int kDtype = GIE_HIP_FP32, kAcc = 4;

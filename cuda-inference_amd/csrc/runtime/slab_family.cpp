@@ -80,7 +80,8 @@ int full_form_of(const Entry& en) {
 
 // Steady-state rate of each form against the split form's, whose profile the family carries (MI355X, FP16 3x3 256 -> 256
 // over 14x14, batch 32 / 288 -> 367 over 12x12, batch 22: split 9.1 / 15.6 us, pipelined 10.3 / 17.7, two lean
-// workgroups a CU 15.1 / 19.8, full 16.0 / 28.8; the full form of the 4- and 8-row slabs is nearer). Taking them for equal made the dispatcher choose the full form.
+// workgroups a CU 15.1 / 19.8, full 16.0 / 28.8; the full form of the 4- and 8-row slabs is nearer). Taking them for equal made the
+// dispatcher choose the full form.
 double rate_of(const gie_slab_config& info) {
   if (info.form == 3) return 1.0;
   if (info.form == 2) return 0.82;

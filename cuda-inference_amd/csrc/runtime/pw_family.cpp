@@ -94,6 +94,41 @@ struct Fns {
   }
   static double extra_traffic(const ConvProblem&) { return 0.0; }  // X, W read and Y written once from HBM
   static int occupancy(const ConvProblem&) { return Stream ? 1 : 2; }
+  // tiles are counted per image, as blocks() does; the streaming form's blocks run over the flat pixel axis
+  static double tile_efficiency(const ConvProblem& prob) {
+    const auto frac = [](int64_t v, int64_t tile) { return double(v) / double((v + tile - 1) / tile * tile); };
+    const Conv2DParams& p = prob.p;
+    const int64_t hw = int64_t(p.in_h) * p.in_w;
+    return frac(p.out_channels, Stream ? 256 : 128) * frac(Stream ? p.batch * hw : hw, Stream ? 64 : 128) *
+           frac(p.in_channels, Stream ? 16 : 32);
+  }
+  // Tiled: fixed cost, then one workgroup's 32-channel steps or a CU's share of the workgroups at a start-up and a cost
+  // for each step. Streaming: the weights (by the k-steps
+  // that their registers hold) once for each round of workgroups an XCD's 32 CUs take, then a CU's 64-pixel blocks.
+  // Both store at a cost for each MB of y, which rises where y leaves the Infinity Cache before the next call writes it.
+  // Fitted to 1076 and 627 layers on one MI355X (7 to 56 a side, 16 to 1024 channels, three sets of tensors in turn):
+  // 13 % and 6 % rms, as much on 82 and 57 others. A FLOP rate put the tiled form first where the streaming one is
+  // faster (256 -> 1024 over 28x28, batch 64: 83.9 and 53.7 us) and the gathering kernel before the tiled form
+  // (512 -> 128 over 28x28, batch 32: 13.2 and 10.3 us).
+  static double busy_us(const ConvProblem& prob, int cus) {
+    const Conv2DParams& p = prob.p;
+    cus = std::max(cus, 1);
+    const double y = double(p.output_shape().numel()) * 2.0 / 1e6;
+    if (!Stream) {
+      const double steps = double((p.in_channels + 31) / 32);
+      const double tiles = double(p.batch) * double((int64_t(p.in_h) * p.in_w + 127) / 128);
+      const double share = tiles * double((p.out_channels + 127) / 128) / cus;
+      return 3.2 + std::max(0.27 * steps, share * (0.1 + 0.32 * steps)) + 0.26 * y + 0.3 * std::max(0.0, y - 60.0);
+    }
+    const int64_t n_ob = (p.out_channels + 255) / 256;
+    const int64_t n_blk = (int64_t(p.batch) * p.in_h * p.in_w + 63) / 64;
+    const int64_t ranges = std::max<int64_t>(1, std::min<int64_t>(n_blk, std::max<int64_t>(1, cus / n_ob)));
+    const int64_t per_xcd = std::max(cus / 8, 1);
+    const double rounds = double(((ranges + 7) / 8 * n_ob + per_xcd - 1) / per_xcd);
+    const double blocks_each = double((n_blk + ranges - 1) / ranges);
+    const double ks = p.in_channels <= 64 ? 4.0 : p.in_channels <= 128 ? 8.0 : 16.0;
+    return 1.3 + rounds * (0.125 * ks + blocks_each * (0.62 + 0.065 * ks)) + 0.11 * y + 0.39 * std::max(0.0, y - 70.0);
+  }
   static void launch(const LaunchArgs& la) {
     const ConvProblem& prob = *la.problem;
     const bool y_ok = Stream ? (reinterpret_cast<uintptr_t>(la.y) & 7u) == 0 : aligned16(la.y);
@@ -131,14 +166,14 @@ KernelDesc make_entry() {
   k.tile_k = Stream ? 16 : 32;
   k.uses_tensor_cores = true;
   k.launches = 1;
-  // the tiled form's rate on 288 and more channels (544 -> 544 over 20x20, batch 3: 9.0 us; the gathering kernel 10.3)
-  if (!Stream) k.relative_rate = 1.2;
   k.supports = &F::supports;
   k.workspace_bytes = &F::workspace;
   k.dynamic_smem_bytes = &F::lds;
   k.num_blocks = &F::blocks;
   k.extra_traffic_bytes = &F::extra_traffic;
   k.blocks_per_cu = &F::occupancy;
+  k.tile_efficiency = &F::tile_efficiency;
+  k.busy_us = &F::busy_us;
   k.launch = &F::launch;
   return k;
 }

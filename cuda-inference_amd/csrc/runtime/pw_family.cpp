@@ -103,11 +103,11 @@ struct Fns {
            frac(p.in_channels, Stream ? 16 : 32);
   }
   // Tiled: fixed cost, then one workgroup's 32-channel steps or a CU's share of the workgroups at a start-up and a cost
-  // for each step. Streaming: the weights (by the k-steps
-  // that their registers hold) once for each round of workgroups an XCD's 32 CUs take, then a CU's 64-pixel blocks.
-  // Both store at a cost for each MB of y, which rises where y leaves the Infinity Cache before the next call writes it.
+  // for each step; its BF16 form rounds with integer arithmetic, which shows as 1.65 us a launch. Streaming: the weights
+  // (by the k-steps that their registers hold) once for each round of workgroups an XCD's 32 CUs take, then a CU's
+  // 64-pixel blocks. Both store at a cost for each MB of y, which rises where y leaves the Infinity Cache before the next call writes it.
   // Fitted to 1076 and 627 layers on one MI355X (7 to 56 a side, 16 to 1024 channels, three sets of tensors in turn):
-  // 13 % and 6 % rms, as much on 82 and 57 others. A FLOP rate put the tiled form first where the streaming one is
+  // 5 % and 6 % rms, as much on 82 and 57 others. A FLOP rate put the tiled form first where the streaming one is
   // faster (256 -> 1024 over 28x28, batch 64: 83.9 and 53.7 us) and the gathering kernel before the tiled form
   // (512 -> 128 over 28x28, batch 32: 13.2 and 10.3 us).
   static double busy_us(const ConvProblem& prob, int cus) {
@@ -118,7 +118,9 @@ struct Fns {
       const double steps = double((p.in_channels + 31) / 32);
       const double tiles = double(p.batch) * double((int64_t(p.in_h) * p.in_w + 127) / 128);
       const double share = tiles * double((p.out_channels + 127) / 128) / cus;
-      return 3.2 + std::max(0.27 * steps, share * (0.1 + 0.32 * steps)) + 0.26 * y + 0.3 * std::max(0.0, y - 60.0);
+      const double bf16 = P == Precision::kBf16 ? 1.0 : 0.0;
+      return 2.25 + 1.65 * bf16 + std::max(0.28 * steps, share * (0.09 + 0.37 * bf16 + 0.34 * steps)) + 0.23 * y +
+             0.3 * std::max(0.0, y - 60.0);
     }
     const int64_t n_ob = (p.out_channels + 255) / 256;
     const int64_t n_blk = (int64_t(p.batch) * p.in_h * p.in_w + 63) / 64;

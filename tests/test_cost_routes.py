@@ -41,10 +41,11 @@ def test_wide_pointwise_layers_take_the_streaming_form(prec, side, batch):
     assert gie.model_rank(p)[0][0] == f"pw_{prec}_1x1_256x64x16_s4_wreg"
 
 
-@pytest.mark.parametrize("case", [(32, 512, 28, 28, 128), (11, 448, 48, 39, 96), (16, 512, 28, 28, 256)],
+@pytest.mark.parametrize("case", [(32, 512, 28, 28, 128), (13, 592, 24, 24, 296), (11, 448, 48, 39, 96), (16, 512, 28, 28, 256)],
                          ids=lambda c: "x".join(map(str, c)))
 def test_pointwise_layers_of_many_channels_take_the_tiled_form(case):
-    """Channels past the streaming form's 256: 10.3, 8.7 and 10.1 us, the gathering kernel 1.26 to 1.31 times those."""
+    """Channels past the streaming form's 256: 10.3, 10.3, 8.7 and 10.1 us, the gathering kernel 1.26 to 1.43 times
+    those."""
     p = P(*case, 1, 1, precision="fp16", has_bias=True, relu=True)
     assert gie.model_rank(p)[0][0] == "pw_fp16_1x1_128x128x32_s4_sk1"
 

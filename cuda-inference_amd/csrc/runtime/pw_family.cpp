@@ -105,31 +105,36 @@ struct Fns {
   // Tiled: fixed cost, then one workgroup's 32-channel steps or a CU's share of the workgroups at a start-up and a cost
   // for each step; its BF16 form rounds with integer arithmetic, which shows as 1.65 us a launch. Streaming: the weights
   // (by the k-steps that their registers hold) once for each round of workgroups an XCD's 32 CUs take, then a CU's
-  // 64-pixel blocks. Both store at a cost for each MB of y, which rises where y leaves the Infinity Cache before the next call writes it.
-  // Fitted to 1076 and 627 layers on one MI355X (7 to 56 a side, 16 to 1024 channels, three sets of tensors in turn):
-  // 5 % and 6 % rms, as much on 82 and 57 others. A FLOP rate put the tiled form first where the streaming one is
-  // faster (256 -> 1024 over 28x28, batch 64: 83.9 and 53.7 us) and the gathering kernel before the tiled form
-  // (512 -> 128 over 28x28, batch 32: 13.2 and 10.3 us).
+  // 64-pixel blocks. Both store at a cost for each MB of y. Where x and y pass 80 MB they no longer stay in the Infinity
+  // Cache between calls on a few sets of tensors, and a MB beyond costs more, most where image rows of y share 128-byte
+  // lines. Fitted to 1316 and 787 layers on one MI355X (7 to 56 a side, 16 to 1024 channels, three sets in turn): 6 % and
+  // 8 % rms, 5 % and 7 % on 82 and 57 others. A FLOP rate put the tiled form first where the streaming one is faster
+  // (256 -> 1024 over 28x28, batch 64: 83.9 and 53.7 us) and the gathering kernel before the tiled form (512 -> 128 over
+  // 28x28, batch 32: 13.2 and 10.3 us).
   static double busy_us(const ConvProblem& prob, int cus) {
     const Conv2DParams& p = prob.p;
     cus = std::max(cus, 1);
-    const double y = double(p.output_shape().numel()) * 2.0 / 1e6;
+    const int64_t hw = int64_t(p.in_h) * p.in_w;
+    const double y = double(p.output_shape().numel()) * 2.0 / 1e6, x = double(p.input_shape().numel()) * 2.0 / 1e6;
+    const double spilled = std::max(0.0, x + y - 80.0);
+    const bool shared_lines = hw % 64 != 0;
     if (!Stream) {
       const double steps = double((p.in_channels + 31) / 32);
-      const double tiles = double(p.batch) * double((int64_t(p.in_h) * p.in_w + 127) / 128);
+      const double tiles = double(p.batch) * double((hw + 127) / 128);
       const double share = tiles * double((p.out_channels + 127) / 128) / cus;
       const double bf16 = P == Precision::kBf16 ? 1.0 : 0.0;
-      return 2.25 + 1.65 * bf16 + std::max(0.28 * steps, share * (0.09 + 0.37 * bf16 + 0.34 * steps)) + 0.23 * y +
-             0.3 * std::max(0.0, y - 60.0);
+      return 2.3 + 1.64 * bf16 + std::max(0.278 * steps, share * (0.21 + 0.46 * bf16 + 0.321 * steps)) + 0.19 * y +
+             (shared_lines ? 0.41 : 0.25) * spilled;
     }
     const int64_t n_ob = (p.out_channels + 255) / 256;
-    const int64_t n_blk = (int64_t(p.batch) * p.in_h * p.in_w + 63) / 64;
+    const int64_t n_blk = (int64_t(p.batch) * hw + 63) / 64;
     const int64_t ranges = std::max<int64_t>(1, std::min<int64_t>(n_blk, std::max<int64_t>(1, cus / n_ob)));
     const int64_t per_xcd = std::max(cus / 8, 1);
     const double rounds = double(((ranges + 7) / 8 * n_ob + per_xcd - 1) / per_xcd);
     const double blocks_each = double((n_blk + ranges - 1) / ranges);
     const double ks = p.in_channels <= 64 ? 4.0 : p.in_channels <= 128 ? 8.0 : 16.0;
-    return 1.3 + rounds * (0.125 * ks + blocks_each * (0.62 + 0.065 * ks)) + 0.11 * y + 0.39 * std::max(0.0, y - 70.0);
+    return 1.45 + rounds * (0.137 * ks + blocks_each * (0.5 + 0.055 * ks)) + 0.111 * y +
+           (shared_lines ? 0.37 : 0.17) * spilled;
   }
   static void launch(const LaunchArgs& la) {
     const ConvProblem& prob = *la.problem;

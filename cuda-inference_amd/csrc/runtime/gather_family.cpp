@@ -78,15 +78,21 @@ struct Fns {
   static int occupancy(const ConvProblem& prob) {
     return std::max<int>(1, std::min<int>(2048 / 2 / tile_of(Config).threads, int(160 * 1024 / std::max<size_t>(lds(prob), 1))));
   }
-  // A workgroup takes `start` us and each 64-channel step `step` us plus a share of its vector loads (16 clocks each: a
-  // wave's x loads cover 64 pixel groups, its w loads 8 rows); one workgroup alone on a CU is bound by latency (`alone`).
-  // Fitted per tile to 58 layers on one MI355X (7 to 56 a side, 14 to 1992 channels, both strides): 11-15 % rms.
+  // A fixed cost (more where images are no multiple of a store's eight pixels), then each 64-channel step at one
+  // workgroup's latency (`alone`) plus, beyond 0.75 workgroups a CU, its share of them (`step`); both grow with the step's
+  // vector loads (16 clocks each: a wave's x loads cover 64 pixel groups, its w loads 8 rows) and where channels end
+  // inside a step (`part`); then the output stores, and more for each MB of x and y past the 80 that stay in the
+  // Infinity Cache over a few sets of tensors (`spill`, `spill_lines` where image rows of y share 128-byte lines). Fitted
+  // per tile to 2106-2199 layers on one MI355X (7 to 56 a side, 16 to 1992 channels, both strides): 8-11 % rms, 8-12 % on
+  // 323-335 others.
   static double busy_us(const ConvProblem& prob, int cus) {
     struct Fit {
-      double fixed, start, step, step_load, alone, alone_load;
+      double fixed, alone, alone_load, step, step_load, out, odd, part, spill, spill_lines;
     };
-    constexpr Fit kFit[] = {{3.4, 0.46, 0.18, 0.93, 0.0, 2.1}, {3.2, 1.33, 0.16, 0.84, 0.23, 1.18},
-                            {4.4, 1.62, 0.69, 0.72, 0.35, 1.19}, {4.0, 4.83, 0.19, 1.52, 0.0, 1.5}};
+    constexpr Fit kFit[] = {{2.07, 0.286, 0.818, 0.148, 0.300, 0.329, 0.89, 0.57, 0.35, 0.28},
+                            {2.24, 0.390, 0.619, 0.290, 0.384, 0.224, 1.04, 0.19, 0.28, 0.19},
+                            {3.07, 0.538, 0.643, 0.456, 0.450, 0.235, 1.52, 0.15, 0.26, 0.14},
+                            {3.16, 0.480, 0.740, 0.169, 1.742, 0.261, 1.37, 0.20, 0.14, 0.16}};
     const Fit& f = kFit[Config];
     const Conv2DParams& p = prob.p;
     const Tile t = tile_of(Config);
@@ -97,8 +103,12 @@ struct Fns {
     const double spread = p.stride_w > 1 ? 1.35 : 1.0;
     const double loads = (spread * double(t.n) / px + t.m / 8.0) * 16.0 / 2400.0;  // us of a step's vector loads
     const double steps = double((p.in_channels + 63) / 64), share = double(blocks(prob)) / std::max(cus, 1);
-    return f.fixed + std::max(steps * (f.alone + f.alone_load * loads),
-                              share * (f.start + steps * (f.step + f.step_load * loads)));
+    const double y = double(p.output_shape().numel()) * 2.0 / 1e6, x = double(p.input_shape().numel()) * 2.0 / 1e6;
+    const int64_t ohw = int64_t(p.out_h()) * p.out_w();
+    const double spill = std::max(0.0, x + y - 80.0) * (f.spill + (ohw % 64 != 0 ? f.spill_lines : 0.0));
+    const double step = f.alone + f.alone_load * loads + std::max(0.0, share - 0.75) * (f.step + f.step_load * loads);
+    const double part = p.in_channels % 64 != 0 ? 1.0 + f.part : 1.0;
+    return f.fixed + (ohw % 8 != 0 ? f.odd : 0.0) + steps * step * part + f.out * y + spill;
   }
   static void launch(const LaunchArgs& la) {
     if (la.only_stage >= 0 && la.only_stage != 1) return;  // one stage: the convolution itself

@@ -10,10 +10,8 @@
 //     expected to be faster: the tile kernel reads each stage one stage ahead and needs hundreds of 64 x 128 tiles,
 //     the other splits the reduction inside a workgroup (one image 3x3 64 -> 64 over 56x56: 6.6 us against 18.3 with
 //     eight split-K slices and their reduce).
-//   * the 128-filter split-8 entry runs whichever of its tile kernel and the padded-NHWC kernel (conv_nhwc.hip) is expected
-//     to be faster, FP32 only and where the copies and partials of the latter fit the entry's own workspace: large layers
-//     (3x3 128 -> 128 over 28x28, batch 32: 92 us against 118 for the 64-filter entry). Here and above the tile kernel keeps
-//     the calls it had: an entry's name, its limits and its workspace do not change.
+//     The tile kernel keeps the calls it had: the entry's name, its limits and its workspace do not change.
+// Large FP32 layers have entries of their own on the padded-NHWC kernel (nhwc_family.cpp).
 // The FP32 matrix-core rate equals the vector FP32 rate on gfx950 (256 FLOP/clk/CU), so the cost model prices
 // these entries against the FP32 ceiling (uses_tensor_cores = false).
 #include <hip/hip_runtime.h>
@@ -25,7 +23,6 @@
 #include "gie_hip.h"
 #include "gpu_inference/kernel_registry.h"
 #include "mini_family.h"
-#include "nhwc_family.h"
 
 namespace gie {
 namespace {
@@ -83,8 +80,7 @@ struct Fns {
   }
   static double extra_traffic(const ConvProblem& prob) {
     // each 128-pixel tile re-reads the weights and each filter tile the activations from L2 (not HBM); split-K
-    // writes and re-reads the FP32 partials. The padded-NHWC kernel's copies are in its own formula.
-    if (nhwc(prob, 256).config >= 0) return 0.0;
+    // writes and re-reads the FP32 partials.
     return Split > 1 ? 2.0 * Split * double(prob.p.output_shape().numel()) * 4.0 : 0.0;
   }
   static int occupancy(const ConvProblem&) { return 2; }
@@ -104,24 +100,13 @@ struct Fns {
     const int c = mini_best_config(prob, cus, &us);
     return c >= 0 && us < tile_us(prob, cus) ? c : -1;
   }
-  // the padded-NHWC configuration that runs this problem in the entry's place (config -1: none)
-  static NhwcF32 nhwc(const ConvProblem& prob, int cus) {
-    if (Split != 8 || tile_m() != 128 || P != Precision::kFp32) return NhwcF32{};
-    const NhwcF32 n = nhwc_f32_best(prob, cus, workspace(prob));
-    return n.config >= 0 && n.us < tile_us(prob, cus) ? n : NhwcF32{};
-  }
   static double busy_us(const ConvProblem& prob, int cus) {
-    if (const NhwcF32 n = nhwc(prob, cus); n.config >= 0) return n.us;
     const int c = mini_config(prob, cus);
     return c >= 0 ? mini_busy_us(c, prob, cus) : tile_us(prob, cus);
   }
   static void launch(const LaunchArgs& la) {
     const ConvProblem& prob = *la.problem;
     const gie_conv_geom g = geom_of(prob);
-    if (const NhwcF32 n = nhwc(prob, la.dev->sm_count); n.config >= 0) {
-      nhwc_f32_launch(n, la);
-      return;
-    }
     float* part = Split > 1 ? static_cast<float*>(la.workspace) : nullptr;
     const auto stage = [&](int k) { return la.only_stage < 0 || la.only_stage == k; };
     // stage 1: the convolution (no repack stage); stage 2: the split-K reduce

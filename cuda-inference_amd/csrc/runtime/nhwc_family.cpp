@@ -1,7 +1,9 @@
 // The padded-NHWC implicit-GEMM family (conv_nhwc.hip: any filter, stride and padding) as registry entries
 // nhwc_<p>_<filters>x<pixels>_sk<S>, in the role of the reference's tcmma registration
 // (src/kernels/tensor_core_mma.cu:264-395): one repack dispatch, the GEMM, and a reduce when split-K.
-//   * capability filter: fp16/bf16, a gfx950 device, offsets, grid and steps within gie_hip_nhwc_check's limits, LDS,
+// FP32 entries (nhwc_fp32_<filters>x<pixels>x32_sk<S>) carry Backend::kImplicitGemm, the reference's FP32 backend, beside the
+// tile kernel's of f32_family.cpp.
+//   * capability filter: fp16/bf16/fp32, a gfx950 device, offsets, grid and steps within gie_hip_nhwc_check's limits, LDS,
 //     workspace at most a quarter of device memory;
 //   * workspace = [padded NHWC x | 256-B align][repacked w | align][split * |Y| FP32 partials | align]. Caller tensors
 //     need only their element's alignment.
@@ -14,7 +16,6 @@
 
 #include "gie_hip.h"
 #include "gpu_inference/kernel_registry.h"
-#include "nhwc_family.h"
 
 namespace gie {
 namespace {
@@ -133,13 +134,19 @@ struct Fns {
     };
     constexpr Fit kFit[] = {{5.2, 0.0, 0.288, 1.09, 0.248}, {6.2, 0.0, 0.368, 1.24, 0.376}, {6.2, 0.4, 0.467, 2.86, 0.654},
                             {6.7, 1.9, 0.750, 4.60, 1.028}, {8.1, 4.2, 1.241, 3.99, 1.865}};
-    const Fit& f = kFit[Config];
     const Plan pl = plan_of(Config, prob);
-    const double share = double(blocks(prob)) / std::max(cus, 1), steps = double(pl.steps) / Split;
-    const double moved = double(pl.x_bytes) + double(prob.p.input_shape().numel()) * 2 + 2.0 * double(pl.w_bytes);
-    const double reduce = Split > 1 ? (Split + 1) * double(prob.p.output_shape().numel()) * 4 / 5e6 : 0.0;
-    return f.fixed + moved / 4.3e6 + reduce +
-           std::max(f.alone + steps * f.alone_step, share * (f.start + steps * f.step));
+    const double steps = double(pl.steps) / Split, share = double(blocks(prob)) / std::max(cus, 1);
+    const double moved = double(pl.x_bytes) + double(prob.p.input_shape().numel()) * double(dtype_size(prob.dtype())) +
+                         2.0 * double(pl.w_bytes);
+    const double partials = Split > 1 ? (Split + 1) * double(prob.p.output_shape().numel()) * 4 / 1e6 : 0.0;  // MB
+    if (P == Precision::kFp32) {
+      // whole rounds of workgroups on CUs that the matrix cores keep busy; fitted to 75 layers (4-7 % rms)
+      constexpr double kFp32[][4] = {{5.2, 0.617, 0.8, 0.526}, {4.5, 1.945, 2.95, 1.945}};  // fixed, alone, start, step
+      const auto& q = kFp32[Config == 0 ? 0 : 1];
+      return q[0] + moved / 4.3e6 + 0.27 * partials + std::max(steps * q[1], std::ceil(share) * (q[2] + steps * q[3]));
+    }
+    const Fit& f = kFit[Config];
+    return f.fixed + moved / 4.3e6 + partials / 5.0 + std::max(f.alone + steps * f.alone_step, share * (f.start + steps * f.step));
   }
   static void launch(const LaunchArgs& la) { run(Config, Split, la); }
 };
@@ -149,16 +156,18 @@ KernelDesc make_entry() {
   using F = Fns<Config, Split, P>;
   const Tile t = tile_of(Config);
   KernelDesc k;
-  k.backend = Backend::kTensorCore;
-  k.name = std::string("nhwc_") + to_string(P) + "_" + std::to_string(t.m) + "x" + std::to_string(t.n) + "x64_sk" +
-           std::to_string(Split);
+  const bool f32 = P == Precision::kFp32;
+  const int bk = f32 ? 32 : 64;  // channels of a step
+  k.backend = f32 ? Backend::kImplicitGemm : Backend::kTensorCore;
+  k.name = std::string("nhwc_") + to_string(P) + "_" + std::to_string(t.m) + "x" + std::to_string(t.n) + "x" +
+           std::to_string(bk) + "_sk" + std::to_string(Split);
   k.version = 1;
-  k.params = {{"block_m", t.m}, {"block_n", t.n}, {"block_k", 64}, {"split_k", Split}};
+  k.params = {{"block_m", t.m}, {"block_n", t.n}, {"block_k", bk}, {"split_k", Split}};
   k.threads_per_block = t.threads;
   k.tile_m = t.m;
   k.tile_n = t.n;
-  k.tile_k = 64;
-  k.uses_tensor_cores = true;
+  k.tile_k = bk;
+  k.uses_tensor_cores = !f32;  // FP32 is priced against the FP32 ceiling, which the FP32 MFMA rate equals
   k.launches = 2 + (Split > 1 ? 1 : 0);
   k.supports = &F::supports;
   k.workspace_bytes = &F::workspace;
@@ -184,43 +193,24 @@ void add_precision(std::vector<KernelDesc>& out) {
   out.push_back(make_entry<2, 2, P>());
 }
 
-}  // namespace
-
-// Per tile: fixed cost, the repack at its traffic, each CU's whole share of the workgroups at a start-up cost and a cost for
-// each 32-channel step, the reduce. Fitted to 75 layers on one MI355X (4-7 % rms).
-NhwcF32 nhwc_f32_best(const ConvProblem& prob, int cus, size_t room) {
-  struct Fit {
-    int config;
-    double fixed, alone_step, start, step;
-  };
-  constexpr Fit kFit[] = {{0, 5.2, 0.617, 0.8, 0.526}, {2, 4.5, 1.945, 2.95, 1.945}};
-  NhwcF32 best;
-  for (const Fit& f : kFit) {
-    const Plan pl = plan_of(f.config, prob);
-    if (!pl.ok) continue;
-    const Tile t = tile_of(f.config);
-    const double y = double(prob.p.output_shape().numel()) * 4;
-    const double moved = double(pl.x_bytes) + double(prob.p.input_shape().numel()) * 4 + 2.0 * double(pl.w_bytes);
-    const int64_t tiles = (prob.p.gemm_n() + t.n - 1) / t.n * ((prob.p.out_channels + t.m - 1) / t.m);
-    for (int split : {1, 2, 4}) {
-      if (split > 1 && pl.steps < 4 * split) continue;
-      const size_t part = split > 1 ? align256(size_t(split) * size_t(y)) : 0;
-      if (align256(pl.x_bytes) + align256(pl.w_bytes) + part > room) continue;
-      const double share = std::ceil(double(tiles * split) / std::max(cus, 1)), steps = double(pl.steps) / split;
-      const double us = f.fixed + moved / 4.3e6 + std::max(steps * f.alone_step, share * (f.start + steps * f.step)) +
-                        (split > 1 ? 1.5 + 0.27 * (split + 1) * y / 1e6 : 0.0);
-      if (best.config < 0 || us < best.us) best.config = f.config, best.split = split, best.us = us;
-    }
-  }
-  return best;
+// FP32: the tiles whose four accumulators fit the registers
+void add_fp32(std::vector<KernelDesc>& out) {
+  constexpr Precision P = Precision::kFp32;
+  out.push_back(make_entry<0, 1, P>());
+  out.push_back(make_entry<2, 1, P>());
+  out.push_back(make_entry<0, 2, P>());
+  out.push_back(make_entry<2, 2, P>());
+  out.push_back(make_entry<0, 4, P>());
+  out.push_back(make_entry<2, 4, P>());
 }
 
-void nhwc_f32_launch(const NhwcF32& how, const LaunchArgs& la) { run(how.config, how.split, la); }
+}  // namespace
 
 void register_nhwc_family(std::vector<KernelDesc>& out) {
   if (gie_hip_nhwc_config_count() != 5) throw Error(StatusCode::kInternal, "padded-NHWC tile table changed");
   add_precision<Precision::kFp16>(out);
   add_precision<Precision::kBf16>(out);
+  add_fp32(out);
 }
 
 }  // namespace gie

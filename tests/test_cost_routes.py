@@ -61,6 +61,20 @@ def test_tiled_pointwise_entry_counts_tiles_per_image():
     assert gie.model_estimate("pw_fp16_1x1_256x64x16_s4_wreg", p)["tile_efficiency"] == 1.0
 
 
+def test_large_fp32_layers_take_entries_that_describe_what_runs():
+    """3x3 128 -> 128 over 28x28, batch 32: the padded-NHWC kernel (90 us; the tile kernel 118) under a name, launches and
+    tiles of its own, and the split-8 tile entry priced as the tile kernel with its eight partials on any device."""
+    p = P(32, 128, 28, 28, 128, 3, 3, 1, 1, 1, 1, precision="fp32", has_bias=True, relu=True)
+    assert gie.model_rank(p)[0][0] == "nhwc_fp32_128x128x32_sk1"
+    d = gie.kernel_describe("nhwc_fp32_128x128x32_sk1")
+    assert (d["backend"], d["launches"], d["threads"], d["tile_m"], d["tile_n"]) == ("implicit_gemm", 2, 512, 128, 128)
+    assert gie.kernel_describe("nhwc_fp32_64x64x32_sk2")["launches"] == 3
+    partials = 2 * 8 * 4 * 32 * 128 * 28 * 28
+    for cus in (64, 128, 256):
+        e = gie.model_estimate("implicit_gemm_fp32_128x128x16_mfma_sk8", p, dict(cus=cus, hbm_gbs=8000.0))
+        assert e["memory_us"] > partials / 8e6
+
+
 @pytest.mark.parametrize("prec", ["fp32", "tf32", "fp16", "bf16"])
 def test_every_estimate_is_finite_and_positive(prec):
     for p in (P(1, 8, 1, 1, 8, 1, 1, 1, 1, 0, 0, precision=prec), P(3, 7, 33, 31, 9, 3, 3, 2, 1, 0, 2, precision=prec),

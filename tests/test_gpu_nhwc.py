@@ -139,18 +139,69 @@ def test_nhwc_fp32(case):
             assert m.passed(), f"config {config} split {split}: {m.summary()}"
 
 
-@pytest.mark.parametrize("case", [(32, 128, 28, 28, 128, 3, 3, 1, 1, 1), (8, 3, 112, 112, 64, 7, 7, 2, 3, 3),
-                                  (2, 24, 9, 9, 32, 3, 3, 1, 1, 1)], ids=lambda c: "x".join(map(str, c)))
-def test_nhwc_fp32_through_the_split_8_entry(case):
-    """The FP32 entry that runs these kernels where they are faster: its workspace is its own eight partials."""
+FP32_LAYERS = [(32, 128, 28, 28, 128, 3, 3, 1, 1, 1), (8, 3, 112, 112, 64, 7, 7, 2, 3, 3), (2, 24, 9, 9, 32, 3, 3, 1, 1, 1)]
+
+
+def _align(n):
+    return (n + 255) // 256 * 256
+
+
+@pytest.mark.parametrize("case", FP32_LAYERS, ids=lambda c: "x".join(map(str, c)))
+def test_nhwc_fp32_entries(case):
+    """The FP32 entries run these kernels (bit for bit the C-ABI's repack, convolution and reduce) in a workspace of their
+    copies and partials alone."""
+    p = gie.Problem(*case[:8], case[7], *case[8:], precision="fp32", has_bias=True, relu=True)
+    b = Bundle(p, 0x8E, O.NORMAL, full_reference=False, sample=4096)
+    g, h, n, t = p.geom(p.in_channels), gie.hip(), int(np.prod(p.y_shape())), b.t
+    ran = 0
+    for name in (k for k in gie.registry() if k.startswith("nhwc_fp32_")):
+        config, split = (0 if "_64x64x" in name else 2), int(name.rsplit("_sk", 1)[1])
+        y, why = run_plan(name, b, repeats=2)
+        if y is None:
+            assert "too short" in why, why
+            continue
+        m = b.compare(y)
+        assert m.passed(), f"{name}: {m.summary()}"
+        xb, wb = ctypes.c_longlong(), ctypes.c_longlong()
+        assert h.gie_hip_nhwc_check(config, 0, ctypes.byref(g), ctypes.byref(xb), ctypes.byref(wb), None, None) == 0
+        part_bytes = 4 * n * split if split > 1 else 0
+        assert gie.Plan(p, name).workspace_bytes == _align(xb.value) + _align(wb.value) + _align(part_bytes)
+        xp, wp = gie.DeviceBuffer(xb.value), gie.DeviceBuffer(wb.value)
+        part = gie.DeviceBuffer(part_bytes) if split > 1 else None
+        t.poison()
+        gie.check_hip(h.gie_hip_repack_nhwc(0, t.dx.addr, xp.addr, t.dw.addr, wp.addr, ctypes.byref(g), None), "repack")
+        gie.check_hip(h.gie_hip_conv_nhwc(config, 0, ctypes.byref(g), xp.addr, wp.addr, t.bias_addr(), t.dy.addr,
+                                          part.addr if part else None, split, None), "conv")
+        if part:
+            gie.check_hip(h.gie_hip_splitk_reduce(0, part.addr, t.bias_addr(), t.dy.addr, n, split, p.out_channels,
+                                                  p.out_h * p.out_w, int(p.relu), None), "reduce")
+        gie.synchronize()
+        assert np.array_equal(y, t.y()), name
+        ran += 1
+    assert ran >= 2
+
+
+@pytest.mark.parametrize("case", FP32_LAYERS, ids=lambda c: "x".join(map(str, c)))
+def test_fp32_split_8_entry_runs_its_own_kernel(case):
+    """Bit for bit gie_hip_conv_f32 with 128 filters a tile and eight splits, in a workspace of eight partials."""
     name = "implicit_gemm_fp32_128x128x16_mfma_sk8"
     p = gie.Problem(*case[:8], case[7], *case[8:], precision="fp32", has_bias=True, relu=True)
     b = Bundle(p, 0x8E, O.NORMAL, full_reference=False, sample=4096)
-    assert gie.Plan(p, name).workspace_bytes == (8 * 4 * int(np.prod(p.y_shape())) + 255) // 256 * 256
+    g, h, n, t = p.geom(p.in_channels), gie.hip(), int(np.prod(p.y_shape())), b.t
+    assert gie.Plan(p, name).workspace_bytes == _align(8 * 4 * n)
     y, why = run_plan(name, b, repeats=2)
     assert y is not None, why
     m = b.compare(y)
     assert m.passed(), m.summary()
+    (config,) = [c for c in range(h.gie_hip_f32_config_count()) if h.gie_hip_f32_config_tile_m(c) == 128]
+    part = gie.DeviceBuffer(8 * 4 * n)
+    t.poison()
+    gie.check_hip(h.gie_hip_conv_f32(config, 0, ctypes.byref(g), t.dx.addr, t.dw.addr, t.bias_addr(), t.dy.addr, part.addr,
+                                     8, None), "conv_f32")
+    gie.check_hip(h.gie_hip_splitk_reduce(0, part.addr, t.bias_addr(), t.dy.addr, n, 8, p.out_channels, p.out_h * p.out_w,
+                                          int(p.relu), None), "reduce")
+    gie.synchronize()
+    assert np.array_equal(y, t.y())
 
 
 def test_nhwc_argument_checks():

@@ -31,6 +31,11 @@ def _us(p):
     (P(16, 704, 17, 17, 1408, 1, 1, precision="bf16"), "gather_bf16_1x1_256x128_t512", "nhwc_bf16_128x256x64_sk1"),
     (P(11, 192, 27, 27, 96, 1, 1, precision="fp16"), "gather_fp16_1x1_64x64_t128", "mini_fp16_32x32_k8w"),
     (P(19, 128, 30, 30, 128, 1, 1, 2, 2, precision="bf16"), "gather_bf16_1x1_64x64_t128", "mini_bf16_32x32_k8w"),
+    # the FP32 tile kernel's rounds, stages and reduce: 55.6 and 78.7 us, 19.6 and 25.8
+    (P(23, 352, 18, 14, 176, 3, 1, 1, 1, 1, 0, precision="tf32", has_bias=False, relu=False), "mfma_tf32_64x128x16_sk8",
+     "mfma_tf32_64x128x16_sk2"),
+    (P(33, 32, 52, 52, 256, 1, 1, 2, 2, precision="fp32"), "implicit_gemm_fp32_64x128x16_mfma_sk1",
+     "implicit_gemm_fp32_128x128x16_mfma_sk1"),
 ])
 def test_measured_order(p, first, second):
     us = _us(p)

@@ -64,37 +64,35 @@ int64_t blocks_of(int config, const ConvProblem& prob) {
 
 }  // namespace
 
-// A CU works through its share of the workgroups at a fixed cost each (pixel set-up, partial tiles, stores) plus a
-// cost for each operand load of its waves. Fitted on one MI355X, 16-bit: 1x1 960 workgroups x 432 loads 17.4 us,
-// x 108 loads 9.9 us; 3x3 1568 x 1296 loads 86 us, 56 x 1296 13.1 us; 7x7 50176 x 108 loads 984 us; FP32 3x3
-// 196 x 360 loads 6.7 us, 3136 x 720 loads 126 us. In FP32 sixteen waves hide the loads of long 1x1 reductions better
-// (800 channels, 15925 pixels: 26 us against 42).
+// One workgroup runs on a CU at a time, so a launch takes whole rounds of them: 1x3 32 -> 32 over 32x32, BF16, takes
+// 5.7 us at 128 to 256 workgroups, 10.0 to 10.2 at 288 to 512, 14.5 at 544 to 640. A round costs `start` (pixel set-up,
+// partial tiles, stores), each operand load of a lane `load` and each superstep of the longest wave's share `step`; with
+// 16x16 tiles over few channels the rounds overlap in part. Strided rows of x take more cache lines (`strided`), odd
+// 16-bit rows of weights element loads (`ragged`). Fitted per type, filter and tile to 95-3907 timings on one MI355X: 5-13 %
+// rms, 5-13 % on 19-720 others.
 double mini_busy_us(int config, const ConvProblem& prob, int cus) {
+  struct Fit {
+    double start, load, step, overlap, strided, ragged;
+  };
+  constexpr Fit kFit[2][3][2] = {  // 16 / 32 bits; 1x1, 3x3, other filters; 16x16, 32x32 tiles
+      {{{1.43, 0.0062, 0.107, 0.47, 0.49, 1.60}, {1.44, 0.0055, 0.332, 0.00, 0.56, 1.77}},
+       {{1.44, 0.0079, 0.082, 0.11, 0.21, 1.37}, {1.48, 0.0073, 0.068, 0.04, 0.31, 1.51}},
+       {{1.63, 0.0061, 0.854, 0.00, 0.00, 1.90}, {2.23, 0.0059, 1.431, 0.00, 0.00, 1.30}}},
+      {{{1.12, 0.0071, 0.579, 0.35, 0.50, 0.00}, {1.39, 0.0102, 0.677, 0.00, 0.40, 0.00}},
+       {{1.81, 0.0096, 0.616, 0.08, 0.24, 0.00}, {2.10, 0.0098, 0.867, 0.09, 0.24, 0.00}},
+       {{1.86, 0.0113, 0.280, 0.00, 0.73, 0.00}, {2.60, 0.0136, 0.455, 0.00, 0.46, 0.00}}}};
   const Conv2DParams& p = prob.p;
   const bool k16 = half_precision(prob.precision), one = p.kernel_h * p.kernel_w == 1;
   const bool nine = p.kernel_h == 3 && p.kernel_w == 3;
-  const int ck = k16 ? 8 : 4, t = tile_of(config);
-  // operand loads of a lane over the reduction's whole supersteps (3x3: 9 chunks of each lane group, else 64 k)
-  const int64_t ss = nine ? 9 * (64 / t) * ck : 8 * ck;
-  const double loads = double((p.gemm_k() + ss - 1) / ss * ss) / (ck * (64 / t)) * (ck + 1);
-  double per_load = !one && !nine ? (t == 16 ? 0.014 : k16 ? 0.0105 : 0.022) : !k16 ? 0.012 : t == 16 && one ? 0.0057 : 0.0085;
-  const double wave = std::max(1.0, double(blocks_of(config, prob)) / std::max(cus, 1));
-  if (waves_of(config) == 16 && (one || nine || wave <= 1.0))
-    per_load *= !one && !nine ? 0.85 : k16 ? 1.0 : one ? 0.7 : 0.95;
-  // weights element by element (3x3, 331 channels: 44 us)
-  if (k16 && p.gemm_k() % 2 != 0) per_load *= one || nine ? 3.5 : 1.4;
-  // strided rows of x take twice the cache lines (1x1 544 -> 32, 29x29 /2, batch 53: 37 us at 16x16)
-  // FP32: 1x1 466 -> 384, 22x22 /2, batch 60: 85 us, twice the unstrided rate's
-  if ((one || (k16 && nine)) && p.stride_w > 1 && wave > 1.0) per_load *= k16 ? 1.6 : 2.0;
-  const double share = k16 ? 0.5 * (wave + std::ceil(wave)) : wave;  // the last wave of workgroups is partly empty
-  // a CU with a single workgroup is bound by its latency, not by its load path (1024 -> 256, 196 pixels: 5.7 us)
-  if (k16 && one && t == 32) per_load -= 0.0038 * std::max(0.0, 2.0 - share);
-  // filters without an unrolled form set up their taps for each workgroup, which a CU with one hides in part (1x3 32 ->
-  // 143 over 43x43: 15 us); 3x3 workgroups beyond two a CU queue on the load path
-  double start = t != 16 ? 1.0 : k16 && one ? 0.7 : 1.3;
-  if (k16 && t == 32 && !one && !nine) start = wave > 1.0 ? 3.6 : 2.2;
-  if (k16 && t == 32 && nine && wave > 2.0) start *= 1.3, per_load *= 1.15;
-  return 0.5 + share * (start + loads * per_load) + (t == 16 ? 0.7 * (share - 1.0) : 0.0);
+  const int ck = k16 ? 8 : 4, t = tile_of(config), nw = waves_of(config);
+  const Fit& f = kFit[k16 ? 0 : 1][one ? 0 : nine ? 1 : 2][t == 16 ? 0 : 1];
+  // supersteps of the reduction (3x3: 9 chunks of each lane group, else 64 k in 16 bits) and a lane's operand loads
+  const int64_t ss = nine ? 9 * (64 / t) * ck : 8 * ck, steps = (p.gemm_k() + ss - 1) / ss;
+  const double loads = double(steps * ss) / (ck * (64 / t)) * (ck + 1);
+  const double share = std::max(1.0, double(blocks_of(config, prob)) / std::max(cus, 1));
+  const double rounds = f.overlap * share + (1.0 - f.overlap) * std::ceil(share);
+  const double spread = p.stride_w > 1 ? 1.0 + f.strided : 1.0, ragged = k16 && p.gemm_k() % 2 != 0 ? 1.0 + f.ragged : 1.0;
+  return rounds * (f.start + loads * f.load * spread * ragged + double((steps + nw - 1) / nw) * f.step);
 }
 
 int mini_best_config(const ConvProblem& prob, int cus, double* us) {

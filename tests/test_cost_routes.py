@@ -31,6 +31,10 @@ def _us(p):
     (P(16, 704, 17, 17, 1408, 1, 1, precision="bf16"), "gather_bf16_1x1_256x128_t512", "nhwc_bf16_128x256x64_sk1"),
     (P(11, 192, 27, 27, 96, 1, 1, precision="fp16"), "gather_fp16_1x1_64x64_t128", "mini_fp16_32x32_k8w"),
     (P(19, 128, 30, 30, 128, 1, 1, 2, 2, precision="bf16"), "gather_bf16_1x1_64x64_t128", "mini_bf16_32x32_k8w"),
+    # small convolutions in whole rounds of workgroups: 7.1 and 10.1 us, 12.9 and 19.7, 6.4 and 9.6
+    (P(16, 32, 12, 12, 128, 1, 3, 1, 1, 0, 1, precision="bf16", relu=False), "nhwc_bf16_64x64x64_sk1", "mini_bf16_32x32_k8w"),
+    (P(26, 416, 33, 33, 32, 1, 1, precision="fp16"), "gather_fp16_1x1_64x128_t256", "mini_fp16_32x32_k8w"),
+    (P(8, 39, 27, 27, 16, 3, 3, 1, 1, 1, 1, precision="bf16"), "mini_bf16_32x32_k8w", "nhwc_bf16_64x64x64_sk1"),
     # the FP32 tile kernel's rounds, stages and reduce: 55.6 and 78.7 us, 19.6 and 25.8
     (P(23, 352, 18, 14, 176, 3, 1, 1, 1, 1, 0, precision="tf32", has_bias=False, relu=False), "mfma_tf32_64x128x16_sk8",
      "mfma_tf32_64x128x16_sk2"),
@@ -64,6 +68,18 @@ def test_tiled_pointwise_entry_counts_tiles_per_image():
     p = P(64, 256, 28, 28, 1024, 1, 1, precision="fp16")
     assert gie.model_estimate("pw_fp16_1x1_128x128x32_s4_sk1", p)["tile_efficiency"] == 784 / (7 * 128)
     assert gie.model_estimate("pw_fp16_1x1_256x64x16_s4_wreg", p)["tile_efficiency"] == 1.0
+
+
+@pytest.mark.parametrize("kh,kw,c,prec,measured", [
+    (1, 3, 32, "bf16", {4: 5.6, 6: 5.7, 8: 5.7, 9: 10.0, 12: 10.1, 16: 10.2, 17: 14.5, 20: 14.5, 24: 14.8}),
+    (3, 3, 64, "bf16", {4: 5.2, 6: 5.2, 8: 5.2, 9: 9.0, 12: 9.0, 16: 9.2, 17: 13.0, 20: 13.0, 24: 13.4})])
+def test_small_convolutions_run_in_whole_rounds_of_workgroups(kh, kw, c, prec, measured):
+    """32 -> 32 or 64 -> 32 over 32x32: 32 workgroups an image, one on each of 256 CUs at a time. The time steps between
+    256 and 288 workgroups and again past 512, and is flat between; the estimate follows it."""
+    for batch, us in measured.items():
+        p = P(batch, c, 32, 32, 32, kh, kw, 1, 1, kh // 2, kw // 2, precision=prec)
+        est = gie.model_estimate(f"mini_{prec}_32x32_k8w", p)["time_us"]
+        assert abs(est / us - 1) < 0.08, (batch, est, us)
 
 
 def test_large_fp32_layers_take_entries_that_describe_what_runs():

@@ -309,8 +309,9 @@ extern "C" int gie_hip_conv_gather(int config, int dtype, const gie_conv_geom* g
   const auto off = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
   if (off(x, 2) || off(w, 2) || off(y, 2) || off(bias, 2)) return GIE_HIP_EINVAL;
   if (off(w, 4)) return GIE_HIP_EUNSUPPORTED;
-  // several pixels per load: stride 1 without padding, whole groups per image, aligned rows
-  const bool flat = g.SH == 1 && g.SW == 1 && g.PH == 0 && g.PW == 0;
+  // several pixels per load: output pixels are the input's (stride 1, no padding, no row or column left out), whole groups
+  // per image, aligned rows
+  const bool flat = g.SH == 1 && g.SW == 1 && g.PH == 0 && g.PW == 0 && gg->out_h == g.H && g.OW == g.W;
   const int px = flat && g.HW % 4 == 0 && !off(x, 8) ? 4 : flat && g.HW % 2 == 0 && !off(x, 4) ? 2 : 1;
   const auto pick = [&](auto e) -> GatherFn {
     using E = decltype(e);

@@ -83,6 +83,25 @@ def test_gather_entry_with_weights_aligned_to_one_element(prec):
     assert m.passed(), m.summary()
 
 
+def test_gather_takes_outputs_smaller_than_the_image():
+    """A geometry whose output leaves out the last rows and columns of a stride-1 layer: output pixels are no longer runs
+    of input pixels, whatever the image size allows."""
+    p = gie.Problem(2, 64, 8, 8, 40, 1, 1, precision="fp16", has_bias=True, relu=False)
+    b = Bundle(p, 0x6F, O.UNIFORM)
+    t, g = b.t, p.geom(64)
+    g.out_h, g.out_w = 5, 6
+    n = 2 * 40 * 5 * 6
+    for config in range(gie.hip().gie_hip_gather_config_count()):
+        _conv(config, p, t, t.dx.addr, t.dw.addr, t.dy.addr)  # every pixel, by wide loads
+        full = t.y()
+        t.poison()
+        gie.check_hip(gie.hip().gie_hip_conv_gather(config, gie.PRECISIONS["fp16"], ctypes.byref(g), t.dx.addr, t.dw.addr,
+                                                    t.bias_addr(), t.dy.addr, None), "conv_gather")
+        gie.synchronize()
+        y = gie.storage_to_float(t.dy.download(np.uint16, n), "fp16").reshape(2, 40, 5, 6)
+        assert np.array_equal(y, full[:, :, :5, :6]), config
+
+
 def test_gather_argument_checks():
     h = gie.hip()
     ok = gie.Problem(1, 16, 5, 5, 16, 1, 1, precision="fp16")

@@ -83,6 +83,26 @@ def test_gather_entry_with_weights_aligned_to_one_element(prec):
     assert m.passed(), m.summary()
 
 
+@pytest.mark.parametrize("c,h,w,stride", [(66, 6, 8, 1), (130, 7, 7, 1), (70, 9, 9, 2), (2, 4, 6, 1)],
+                         ids=lambda v: str(v))
+def test_gather_ignores_what_lies_past_the_reduction(c, h, w, stride):
+    """Channels end inside a 16-byte chunk of weights that runs into the next filter. Every second filter and the next
+    image are infinite: nothing of them may reach the others' sums, not even times the zeros that x is past its channels."""
+    p = gie.Problem(2, c, h, w, 20, 1, 1, stride, stride, precision="fp16", has_bias=False, relu=False)
+    b = Bundle(p, 0x6D, O.UNIFORM)
+    x, wt = b.x.copy(), b.w.copy()
+    x[1] = np.inf
+    wt[1::2] = np.inf
+    t = gie.ConvTensors(p, x, wt, None)
+    for config in range(gie.hip().gie_hip_gather_config_count()):
+        _conv(config, p, b.t, b.t.dx.addr, b.t.dw.addr, b.t.dy.addr)
+        ref = b.t.y()
+        t.poison()
+        _conv(config, p, t, t.dx.addr, t.dw.addr, t.dy.addr)
+        y = t.y()
+        assert np.isfinite(y[0, ::2]).all() and np.array_equal(y[0, ::2], ref[0, ::2]), config
+
+
 def test_gather_takes_outputs_smaller_than_the_image():
     """A geometry whose output leaves out the last rows and columns of a stride-1 layer: output pixels are no longer runs
     of input pixels, whatever the image size allows."""

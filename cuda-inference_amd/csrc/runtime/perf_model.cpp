@@ -7,7 +7,9 @@
 //   fixed   = launches x dispatch cost + the family's cost of filling and draining a launch
 //   serial  = passes that do not overlap the main kernel (KernelDesc::serial_us: a repack, a reduce)
 //   time    = max(compute, memory) + fixed + serial  (reported as launch_us; "launch"-bound when it dominates)
-// A family with a formula of its own (KernelDesc::busy_us: everything but dispatch) takes that as its compute time.
+// A family with a formula of its own (KernelDesc::busy_us: everything but dispatch) is timed as max(busy, memory) +
+// dispatch; compute, memory and fixed stay the roofline's parts, by which the estimate is called compute-, bandwidth- or
+// launch-bound.
 // * Family efficiencies are not guesses per backend: each is what that kernel family reached on an MI355X in the
 //   library's benchmark protocol (per-call time, inputs resident in HBM), listed in kFamilies with the measurement.
 // * Wave efficiency follows how gfx950 places workgroups: dispatch deals them round-robin to the 8 XCDs, and each
@@ -68,10 +70,10 @@ constexpr FamilyProfile kFamilies[] = {
     {"stack_", 0.33, 0.40, 4.1},    // L5 9.6 us at split 2 (6.7 conv + 2.8 reduce), 10.2 at split 1
     {"deep_", 0.44, 0.40, 2.9},     // L5 6.6 us: steps at 0.44 of peak, ~4.2 us of set-up, first stage and
                                     // partial-tile exchange per unit
-    // families with a formula of their own: only the bandwidth is used
-    {"mini_", 0.30, 0.50, 0.0},     // its cases are far below the bandwidth
-    {"nhwc_", 0.30, 0.50, 0.0},     // BF16 3x3 64 -> 64, 56x56, batch 32: 28.7 us = 2.7 TB/s with the repack's copy
-    {"gather_", 0.30, 0.50, 0.0},   // 1x1 256 -> 128, 56x56, batch 32: 23.2 us = 3.3 TB/s; at /2 to 512: 2.7 TB/s
+    // families whose time is a formula of their own from the start: the rate only tells what bounds a call
+    {"mini_", 0.30, 0.50, 1.5},     // its cases are far below the bandwidth
+    {"nhwc_", 0.30, 0.50, 5.0},     // BF16 3x3 64 -> 64, 56x56, batch 32: 28.7 us = 2.7 TB/s with the repack's copy
+    {"gather_", 0.30, 0.50, 2.0},   // 1x1 256 -> 128, 56x56, batch 32: 23.2 us = 3.3 TB/s; at /2 to 512: 2.7 TB/s
     {"f32_", 0.30, 0.35, 2.0},      // FP32 / TF32 vector kernels: not benchmarked, assumed
 };
 
@@ -306,22 +308,25 @@ Estimate estimate_kernel(const ConvProblem& prob, const KernelDesc& k, const Dev
   const double peak_tflops = k.uses_tensor_cores ? c.fp16_tc_tflops : c.fp32_tflops;
   const double rate = peak_tflops * 1e6 * mfma_eff * k.relative_rate * std::max(e.tile_efficiency, 1e-3) *
                       std::max(e.wave_efficiency, 1e-3);  // FLOP per us
-  e.compute_us = k.busy_us ? k.busy_us(prob, dev.sm_count) : m.flops / rate;
+  e.compute_us = m.flops / rate;
+  double busy_us = k.busy_us ? k.busy_us(prob, dev.sm_count) : e.compute_us;
   const double traffic = m.compulsory_bytes + (k.extra_traffic_bytes ? k.extra_traffic_bytes(prob) : 0.0);
   e.memory_us = traffic / (c.bw_gbs * 1e3 * hbm_eff);
   // resident workgroups overlap each other's set-up, so only the launch's first fill and last drain are exposed
-  e.launch_us = c.launch_overhead_us * std::max(k.launches, 1) +
-                (k.busy_us ? 0.0 : fam ? fam->fill_us : 2.0);
+  const double dispatch_us = c.launch_overhead_us * std::max(k.launches, 1);
+  e.launch_us = dispatch_us + (fam ? fam->fill_us : 2.0);
   {
     std::lock_guard<std::mutex> lock(g_scale_mu);
     const auto it = backend_scale().find(to_string(k.backend));
     if (it != backend_scale().end()) {
       e.compute_us *= it->second;
       e.memory_us *= it->second;
+      busy_us *= it->second;
     }
   }
   e.bound = bound_of(e.compute_us, e.memory_us, e.launch_us);
-  e.time_us = std::max(e.compute_us, e.memory_us) + e.launch_us + (k.serial_us ? k.serial_us(prob) : 0.0);
+  e.time_us = std::max(busy_us, e.memory_us) + (k.busy_us ? dispatch_us : e.launch_us) +
+              (k.serial_us ? k.serial_us(prob) : 0.0);
   return e;
 }
 

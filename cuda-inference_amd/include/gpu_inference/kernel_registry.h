@@ -71,7 +71,8 @@ struct KernelDesc {
   // Resident workgroups per CU of the main kernel (MI355X-specific addition; null -> 1).
   int (*blocks_per_cu)(const ConvProblem&) = nullptr;
   // Modeled time (us) of the main kernel on `cus` CUs beyond its dispatch, for a family whose time follows a formula of
-  // its own; the cost model takes it in place of FLOPs over a rate (MI355X-specific addition; null -> FLOP rate).
+  // its own; the cost model times the kernel by it in place of FLOPs over a rate (MI355X-specific addition; null -> FLOP
+  // rate).
   double (*busy_us)(const ConvProblem&, int cus) = nullptr;
   // Modeled time (us) of passes before or after the main kernel that do not overlap it (MI355X-specific addition).
   double (*serial_us)(const ConvProblem&) = nullptr;

@@ -43,8 +43,8 @@ struct ProblemModel {
 ProblemModel analyze_problem(const ConvProblem& prob);
 
 struct Estimate {
-  double time_us = 0;
-  double compute_us = 0, memory_us = 0, launch_us = 0;
+  double time_us = 0;  // by the kernel's own formula where it has one, else max(compute, memory) + launch
+  double compute_us = 0, memory_us = 0, launch_us = 0;  // the roofline's parts
   Bound bound = Bound::kCompute;
   double tile_efficiency = 1.0;
   double wave_efficiency = 1.0;  // workgroup load balance over CUs

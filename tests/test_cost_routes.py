@@ -96,6 +96,18 @@ def test_large_fp32_layers_take_entries_that_describe_what_runs():
         assert e["memory_us"] > partials / 8e6
 
 
+@pytest.mark.parametrize("kernel,p,bound", [
+    ("gather_fp16_1x1_64x64_t128", P(1, 8, 4, 4, 8, 1, 1, precision="fp16"), "launch"),
+    ("gather_fp16_1x1_64x64_t128", P(32, 8, 224, 224, 8, 1, 1, precision="fp16"), "bandwidth"),
+    ("band_fp16_3x3_32x256x32_s3_sk1", P(1, 8, 8, 8, 8, 3, 3, 1, 1, 1, 1, precision="fp16"), "launch"),
+    ("halo_fp16_3x3_64x128x32_s2_sk1", P(1, 8, 8, 8, 8, 3, 3, 1, 1, 1, 1, precision="fp16"), "launch"),
+    ("nhwc_bf16_256x256x64_sk1", P(16, 256, 56, 56, 256, 3, 3, 1, 1, 1, 1, precision="bf16"), "compute"),
+])
+def test_estimates_name_what_bounds_a_call(kernel, p, bound):
+    """Entries timed by a formula of their own keep the roofline's parts: a formula's fixed costs are not arithmetic."""
+    assert gie.model_estimate(kernel, p)["bound"] == bound
+
+
 @pytest.mark.parametrize("prec", ["fp32", "tf32", "fp16", "bf16"])
 def test_every_estimate_is_finite_and_positive(prec):
     for p in (P(1, 8, 1, 1, 8, 1, 1, 1, 1, 0, 0, precision=prec), P(3, 7, 33, 31, 9, 3, 3, 2, 1, 0, 2, precision=prec),

@@ -31,6 +31,10 @@ def _us(p):
     (P(16, 704, 17, 17, 1408, 1, 1, precision="bf16"), "gather_bf16_1x1_256x128_t512", "nhwc_bf16_128x256x64_sk1"),
     (P(11, 192, 27, 27, 96, 1, 1, precision="fp16"), "gather_fp16_1x1_64x64_t128", "mini_fp16_32x32_k8w"),
     (P(19, 128, 30, 30, 128, 1, 1, 2, 2, precision="bf16"), "gather_bf16_1x1_64x64_t128", "mini_bf16_32x32_k8w"),
+    # the implicit GEMM over images of no multiple of four pixels: 20.3 and 31.2 us, 47.2 and 78.3; its tiles: 31.2 and 26.2
+    (P(4, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x64x32_w2x2_s4_sk1"),
+    (P(14, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x128x32_w2x2_s4_sk1"),
+    (P(4, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "mfma_fp16_128x128x32_w2x2_s4_sk1", "mfma_fp16_64x64x32_w2x2_s4_sk1"),
     # small convolutions in whole rounds of workgroups: 7.1 and 10.1 us, 12.9 and 19.7, 6.4 and 9.6
     (P(16, 32, 12, 12, 128, 1, 3, 1, 1, 0, 1, precision="bf16", relu=False), "nhwc_bf16_64x64x64_sk1", "mini_bf16_32x32_k8w"),
     (P(26, 416, 33, 33, 32, 1, 1, precision="fp16"), "gather_fp16_1x1_64x128_t256", "mini_fp16_32x32_k8w"),

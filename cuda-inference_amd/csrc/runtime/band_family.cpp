@@ -108,14 +108,18 @@ struct Fns {
     if (gie_hip_band_check(e().config, &g, &bytes) != GIE_HIP_OK) return 0;
     return size_t(bytes);
   }
+  // output rows of a band: rows of a power-of-two padded width in tile_n positions
+  static int rows_of(const ConvProblem& prob) {
+    int owp = 1;
+    while (owp < prob.p.out_w()) owp *= 2;
+    return std::max(1, e().info.tile_n / owp);
+  }
   // Useful output positions of a workgroup's tile_n-position band (rows of a power-of-two padded width, one image
   // per band), times the filter and channel padding.
   static double tile_efficiency(const ConvProblem& prob) {
     const Entry& en = e();
     const Conv2DParams& p = prob.p;
-    int owp = 1;
-    while (owp < p.out_w()) owp *= 2;
-    const int rows = std::max(1, en.info.tile_n / owp);
+    const int rows = rows_of(prob);
     const int64_t bands = (p.out_h() + rows - 1) / rows;
     const double pos = double(p.out_h()) * p.out_w() / (double(bands) * en.info.tile_n);
     const double o = double(p.out_channels) / double(((p.out_channels + en.info.tile_m - 1) / en.info.tile_m) *
@@ -128,9 +132,7 @@ struct Fns {
     // one workgroup per (32 output channels, image, band of rows); a band is tile_n / padded-row-width rows
     const Entry& en = e();
     const Conv2DParams& p = prob.p;
-    int owp = 1;
-    while (owp < p.out_w()) owp *= 2;
-    const int rows = std::max(1, en.info.tile_n / owp);
+    const int rows = rows_of(prob);
     const int64_t bands = (p.out_h() + rows - 1) / rows;
     return int64_t((p.out_channels + en.info.tile_m - 1) / en.info.tile_m) * p.batch * bands * en.split;
   }
@@ -147,21 +149,28 @@ struct Fns {
     const size_t l = lds(prob);
     return l > 80 * 1024 ? 1 : 2;
   }
-  // Fixed cost, the weight repack, a CU's share of the workgroups at a start-up cost and a cost for each 32-channel
-  // slice (or one workgroup's latency), the output's half-empty store runs, and the reduce. Fitted to 69-91 layers per
-  // tile on one MI355X (15-19 % rms); a FLOP rate and bytes missed by up to 2.5x on images of 28 and more a side.
+  // Fixed cost, the weight repack, one workgroup's latency or a CU's share of the workgroups at a start-up cost, each
+  // 32-channel slice at a cost of its own and for the input pixels of a band that it loads (a stride doubles their rows),
+  // output stores, and the reduce. Fitted to 1045 and 775 timings on one MI355X: 13 % and 11 % rms, as much on 585 others;
+  // without the band's pixels 20 % and 18 %, up to 1.6x at stride 2.
   static double busy_us(const ConvProblem& prob, int cus) {
+    struct Fit {
+      double fixed, weights, alone, slice, pixels, start, share_slice, share_pixels, out, reduce;
+    };
     const Entry& en = e();
-    const bool wide = en.info.tile_n == 256;
+    const Fit f = en.info.tile_n == 256 ? Fit{2.34, 1.08, 3.16, 0.50, 0.65, 4.72, 0.42, 0.68, 0.10, 0.33}
+                                        : Fit{2.84, 0.79, 2.43, 0.54, 0.67, 3.94, 0.78, 0.59, 0.00, 0.28};
+    const Conv2DParams& p = prob.p;
     const double slices = double(slices_of(prob, en)) / en.split;
     const double rounds = double(blocks(prob)) / std::max(cus, 1);
     const double share = 0.5 * (rounds + std::ceil(rounds));  // the last round is partly empty
-    const double y = double(prob.p.output_shape().numel()) / 1e6;  // million outputs
-    const double wp = double(prob.p.out_channels) * prob.p.kernel_h * prob.p.kernel_w * c_pad_of(prob) * 2.0 / 1e6;
-    const double reduce = en.split > 1 ? (en.split + 1) * 4.0 * y * (wide ? 0.47 : 0.26) : 0.0;
-    const double alone = wide ? 1.3 + 1.56 * slices : 1.42 * slices;
-    const double shared = share * (wide ? 2.2 + 1.44 * slices : 4.1 + 0.95 * slices);
-    return (wide ? 3.7 : 5.1) + 2.0 * wp / 4.3 + std::max(alone, shared) + y * (wide ? 3.5 : 1.44) + reduce;
+    const double pixels = std::min(double(p.in_h), double(rows_of(prob)) * p.stride_h + p.kernel_h - 1) * p.in_w / 100.0;
+    const double y = double(p.output_shape().numel()) * 2.0 / 1e6;  // MB
+    const double wp = double(p.out_channels) * p.kernel_h * p.kernel_w * c_pad_of(prob) * 2.0 / 1e6;
+    const double reduce = en.split > 1 ? f.reduce * (en.split + 1) * 2.0 * y : 0.0;
+    return f.fixed + f.weights * wp + f.out * y + reduce +
+           std::max(f.alone + (f.slice + f.pixels * pixels) * slices,
+                    share * (f.start + (f.share_slice + f.share_pixels * pixels) * slices));
   }
   static void launch(const LaunchArgs& la) {
     const Entry& en = e();

@@ -31,6 +31,10 @@ def _us(p):
     (P(16, 704, 17, 17, 1408, 1, 1, precision="bf16"), "gather_bf16_1x1_256x128_t512", "nhwc_bf16_128x256x64_sk1"),
     (P(11, 192, 27, 27, 96, 1, 1, precision="fp16"), "gather_fp16_1x1_64x64_t128", "mini_fp16_32x32_k8w"),
     (P(19, 128, 30, 30, 128, 1, 1, 2, 2, precision="bf16"), "gather_bf16_1x1_64x64_t128", "mini_bf16_32x32_k8w"),
+    # a band's input pixels: 58.7 and 110.5 us, 15.2 and 22.8 (stride 2)
+    (P(15, 352, 32, 32, 272, 3, 3, 1, 1, 1, 1, precision="bf16", has_bias=False, relu=False), "nhwc_bf16_128x256x64_sk1",
+     "band_bf16_3x3_32x224x32_s4_sk1"),
+    (P(6, 256, 33, 33, 64, 3, 3, 2, 2, 1, 1, precision="bf16"), "nhwc_bf16_64x64x64_sk4", "band_bf16_3x3_32x256x32_s3_sk4"),
     # the implicit GEMM over images of no multiple of four pixels: 20.3 and 31.2 us, 47.2 and 78.3; its tiles: 31.2 and 26.2
     (P(4, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x64x32_w2x2_s4_sk1"),
     (P(14, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x128x32_w2x2_s4_sk1"),

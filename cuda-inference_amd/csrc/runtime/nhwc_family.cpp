@@ -125,28 +125,36 @@ struct Fns {
   static int occupancy(const ConvProblem& prob) {
     return std::max<int>(1, std::min<int>(2048 / tile_of(Config).threads, int(160 * 1024 / std::max<size_t>(lds(prob), 1))));
   }
-  // Fixed cost (two launches' set-up and drain, dispatch aside), the repack and the reduce at their traffic, then each
-  // CU's share of the workgroups at a start-up cost and a cost for each 64-element step, or one workgroup's latency
-  // where there are fewer than CUs. Fitted per tile to 120-229 layers on one MI355X: 9-13 % rms.
+  // Fixed cost (two launches' set-up and drain, dispatch aside; more where images of x are no multiple of four pixels or
+  // images of y of eight), the repack of x and w, the output and the reduce at their traffic, then one workgroup's latency
+  // or each CU's share of the workgroups (the last round partly empty) at a start-up cost and a cost for each step of 64
+  // 16-bit units. Fitted per tile to 894-4825 timings on one MI355X: 6-8 % rms, 6-8 % on held-out layers (11-17 % without
+  // the odd images and the rounds). FP32: 555 and 467 timings, 8 % and 6 %.
   static double busy_us(const ConvProblem& prob, int cus) {
     struct Fit {
-      double fixed, alone, alone_step, start, step;
+      double fixed, alone, alone_step, start, step, x, w, reduce, out, odd_x, odd_y;
     };
-    constexpr Fit kFit[] = {{5.2, 0.0, 0.288, 1.09, 0.248}, {6.2, 0.0, 0.368, 1.24, 0.376}, {6.2, 0.4, 0.467, 2.86, 0.654},
-                            {6.7, 1.9, 0.750, 4.60, 1.028}, {8.1, 4.2, 1.241, 3.99, 1.865}};
+    constexpr Fit kFit[] = {{3.06, 0.49, 0.272, 1.01, 0.198, 0.254, 0.87, 0.252, 0.164, 0.86, 0.71},
+                            {3.97, 0.43, 0.346, 0.80, 0.308, 0.247, 0.94, 0.266, 0.204, 0.91, 1.01},
+                            {2.98, 1.73, 0.434, 2.28, 0.533, 0.235, 0.98, 0.257, 0.222, 0.92, 1.25},
+                            {3.48, 2.82, 0.733, 3.13, 0.989, 0.217, 1.19, 0.000, 0.152, 0.90, 2.27},
+                            {3.52, 4.79, 1.188, 4.69, 1.483, 0.206, 1.75, 0.000, 0.145, 1.41, 4.03}};
+    constexpr Fit kFp32[] = {{3.35, 0.78, 0.642, 1.08, 0.597, 0.187, 0.79, 0.248, 0.120, 0.0, 0.0},
+                             {3.07, 2.44, 2.043, 2.92, 2.107, 0.187, 1.17, 0.286, 0.196, 0.0, 0.0}};
+    constexpr bool f32 = P == Precision::kFp32;
+    const Fit& f = f32 ? kFp32[Config == 0 ? 0 : 1] : kFit[Config];
+    const Conv2DParams& p = prob.p;
     const Plan pl = plan_of(Config, prob);
-    const double steps = double(pl.steps) / Split, share = double(blocks(prob)) / std::max(cus, 1);
-    const double moved = double(pl.x_bytes) + double(prob.p.input_shape().numel()) * double(dtype_size(prob.dtype())) +
-                         2.0 * double(pl.w_bytes);
-    const double partials = Split > 1 ? (Split + 1) * double(prob.p.output_shape().numel()) * 4 / 1e6 : 0.0;  // MB
-    if (P == Precision::kFp32) {
-      // whole rounds of workgroups on CUs that the matrix cores keep busy; fitted to 75 layers (4-7 % rms)
-      constexpr double kFp32[][4] = {{5.2, 0.617, 0.8, 0.526}, {4.5, 1.945, 2.95, 1.945}};  // fixed, alone, start, step
-      const auto& q = kFp32[Config == 0 ? 0 : 1];
-      return q[0] + moved / 4.3e6 + 0.27 * partials + std::max(steps * q[1], std::ceil(share) * (q[2] + steps * q[3]));
-    }
-    const Fit& f = kFit[Config];
-    return f.fixed + moved / 4.3e6 + partials / 5.0 + std::max(f.alone + steps * f.alone_step, share * (f.start + steps * f.step));
+    const double es = double(dtype_size(prob.dtype()));
+    const double steps = double(pl.steps) / Split, rounds = double(blocks(prob)) / std::max(cus, 1);
+    const double whole = f32 ? 0.87 : 0.5;  // weight of whole rounds: FP32 steps keep the matrix cores busy
+    const double share = (1.0 - whole) * rounds + whole * std::ceil(rounds);
+    const double x = (double(pl.x_bytes) + double(p.input_shape().numel()) * es) / 1e6, w = 2.0 * double(pl.w_bytes) / 1e6;
+    const double y = double(p.output_shape().numel()) * es / 1e6;
+    const double partials = Split > 1 ? (Split + 1) * double(p.output_shape().numel()) * 4.0 / 1e6 : 0.0;  // MB, as the above
+    const bool odd_x = int64_t(p.in_h) * p.in_w % 4 != 0, odd_y = int64_t(p.out_h()) * p.out_w() % 8 != 0;
+    return f.fixed + (odd_x ? f.odd_x : 0.0) + (odd_y ? f.odd_y : 0.0) + f.x * x + f.w * w + f.out * y + f.reduce * partials +
+           std::max(f.alone + steps * f.alone_step, share * (f.start + steps * f.step));
   }
   static void launch(const LaunchArgs& la) { run(Config, Split, la); }
 };

@@ -31,6 +31,10 @@ def _us(p):
     (P(16, 704, 17, 17, 1408, 1, 1, precision="bf16"), "gather_bf16_1x1_256x128_t512", "nhwc_bf16_128x256x64_sk1"),
     (P(11, 192, 27, 27, 96, 1, 1, precision="fp16"), "gather_fp16_1x1_64x64_t128", "mini_fp16_32x32_k8w"),
     (P(19, 128, 30, 30, 128, 1, 1, 2, 2, precision="bf16"), "gather_bf16_1x1_64x64_t128", "mini_bf16_32x32_k8w"),
+    # the padded-NHWC kernel's rounds, stores and odd images: 28.8 and 48.7 us, 24.9 and 40.3, 19.0 and 25.5
+    (P(39, 32, 36, 36, 1024, 1, 1, precision="fp16"), "pw_fp16_1x1_256x64x16_s4_wreg", "nhwc_fp16_256x256x64_sk1"),
+    (P(24, 48, 36, 56, 1024, 1, 1, precision="fp16"), "pw_fp16_1x1_256x64x16_s4_wreg", "nhwc_fp16_256x256x64_sk1"),
+    (P(11, 416, 15, 15, 1664, 1, 1, precision="bf16"), "gather_bf16_1x1_256x128_t512", "nhwc_bf16_128x128x64_sk1"),
     # a band's input pixels: 58.7 and 110.5 us, 15.2 and 22.8 (stride 2)
     (P(15, 352, 32, 32, 272, 3, 3, 1, 1, 1, 1, precision="bf16", has_bias=False, relu=False), "nhwc_bf16_128x256x64_sk1",
      "band_bf16_3x3_32x224x32_s4_sk1"),

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <string>
 #include <vector>
 
@@ -125,25 +126,31 @@ struct Fns {
     const size_t l = lds(prob);
     return l > 80 * 1024 ? 1 : 2;
   }
-  // Fixed cost, the repack at `traffic` us/MB, a CU's share of the workgroups at a start-up cost and a cost for each
-  // 32-channel slice (or one workgroup's latency), output stores, and the reduce. Fitted to 20-125 layers per tile on one
-  // MI355X (7-12 % rms); a FLOP rate missed by up to 2x on images of 20 and more a side with few channels.
+  // Fixed cost (more where images of x are no multiple of four pixels, which the repack takes element by element), the
+  // repack, the output (more where images of y are no multiple of eight) and the reduce at their traffic, then one
+  // workgroup's latency or a CU's share of the workgroups (the last round partly empty) at a start-up cost and a cost for
+  // each 32-channel slice. Fitted per tile to 191-2201 timings on one MI355X: 5-10 % rms, 7-9 % on held-out layers (11-19 %
+  // without the odd images and the rounds).
   static double busy_us(const ConvProblem& prob, int cus) {
     struct Fit {
-      double fixed, alone, alone_slice, start, slice, out, reduce, traffic;
+      double fixed, alone, alone_slice, start, slice, x, w, reduce, out, odd_x, odd_out;
     };
     const Entry& en = e();
-    const Fit f = en.info.kernel_h > 1 ? en.info.stages == 2 ? Fit{4.9, 1.8, 0.98, 5.3, 0.92, 0.59, 0.31, 0.57}
-                                                             : Fit{5.9, 1.8, 0.45, 2.7, 0.58, 0.0, 0.49, 0.97}
-                  : en.info.tile_m == 64 ? Fit{6.4, 0.0, 0.24, 1.4, 0.18, 0.68, 0.31, 0.39}
-                                         : Fit{8.6, 0.7, 0.37, 6.9, 0.21, 0.43, 0.25, 0.28};
+    const Fit f = en.info.kernel_h > 1
+                      ? en.info.stages == 2 ? Fit{3.72, 2.45, 1.04, 4.75, 1.34, 0.308, 0.371, 0.406, 0.00, 1.62, 0.21}
+                                            : Fit{4.15, 2.32, 0.80, 5.01, 1.18, 0.387, 0.375, 0.455, 0.00, 1.47, 0.00}
+                  : en.info.tile_m == 64 ? Fit{4.06, 0.73, 0.30, 2.63, 0.21, 0.395, 0.621, 0.346, 0.01, 2.33, 0.24}
+                                         : Fit{2.13, 5.61, 0.39, 7.89, 0.36, 0.298, 0.437, 0.419, 0.22, 3.79, 0.30};
+    const Conv2DParams& p = prob.p;
     const double slices = double(slices_of(prob, en)) / en.split;
-    const double share = double(blocks(prob)) / std::max(cus, 1);
-    const double y = double(prob.p.output_shape().numel()) / 1e6;  // million outputs
-    const double moved = (double(prob.p.batch) * prob.p.in_h * prob.p.in_w +
-                          double(prob.p.out_channels) * prob.p.kernel_h * prob.p.kernel_w) * c_pad_of(prob) * 4.0 / 1e6;
-    const double reduce = en.split > 1 ? (en.split + 1) * 4.0 * y * f.reduce : 0.0;
-    return f.fixed + moved * f.traffic + y * f.out + reduce +
+    const double rounds = double(blocks(prob)) / std::max(cus, 1), share = 0.5 * (rounds + std::ceil(rounds));
+    const double cp = c_pad_of(prob), taps = double(p.kernel_h) * p.kernel_w;
+    const double x = double(p.batch) * p.in_h * p.in_w * (p.in_channels + cp) * 2.0 / 1e6;  // MB, as the others
+    const double w = double(p.out_channels) * taps * cp * 4.0 / 1e6;
+    const double y = double(p.output_shape().numel()) * 2.0 / 1e6;
+    const bool odd_x = int64_t(p.in_h) * p.in_w % 4 != 0, odd_y = int64_t(p.out_h()) * p.out_w() % 8 != 0;
+    const double reduce = en.split > 1 ? f.reduce * (en.split + 1) * 2.0 * y : 0.0;
+    return f.fixed + (odd_x ? f.odd_x : 0.0) + f.x * x + f.w * w + (f.out + (odd_y ? f.odd_out : 0.0)) * y + reduce +
            std::max(f.alone + f.alone_slice * slices, share * (f.start + f.slice * slices));
   }
   static void launch(const LaunchArgs& la) {

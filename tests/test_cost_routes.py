@@ -35,6 +35,9 @@ def _us(p):
     (P(39, 32, 36, 36, 1024, 1, 1, precision="fp16"), "pw_fp16_1x1_256x64x16_s4_wreg", "nhwc_fp16_256x256x64_sk1"),
     (P(24, 48, 36, 56, 1024, 1, 1, precision="fp16"), "pw_fp16_1x1_256x64x16_s4_wreg", "nhwc_fp16_256x256x64_sk1"),
     (P(11, 416, 15, 15, 1664, 1, 1, precision="bf16"), "gather_bf16_1x1_256x128_t512", "nhwc_bf16_128x128x64_sk1"),
+    # the halo kernel's rounds, repack and odd images: 24.9 and 33.8 us, 32.2 and 42.7
+    (P(4, 160, 53, 53, 160, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_128x128x64_sk1", "halo_bf16_3x3_64x128x32_s2_sk1"),
+    (P(6, 256, 39, 39, 256, 3, 3, 1, 1, 1, 1, precision="fp16"), "nhwc_fp16_128x128x64_sk1", "halo_fp16_3x3_64x128x32_s2_sk1"),
     # a band's input pixels: 58.7 and 110.5 us, 15.2 and 22.8 (stride 2)
     (P(15, 352, 32, 32, 272, 3, 3, 1, 1, 1, 1, precision="bf16", has_bias=False, relu=False), "nhwc_bf16_128x256x64_sk1",
      "band_bf16_3x3_32x224x32_s4_sk1"),

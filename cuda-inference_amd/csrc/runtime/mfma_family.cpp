@@ -79,34 +79,34 @@ std::vector<Entry>& entries() {
 
 // Time of a launch beyond its dispatches, per tile and wave layout: a fixed cost (more where images of x or y are no
 // multiple of four pixels, which the repack and the stores take element by element), `first` for a CU's share of the
-// workgroups, `alone` for each K step of one workgroup and `more` for each step of the share past the first; the repack,
-// the output and the reduce at their traffic, common to all. Fitted to 37 828 timings of 3044 layers on one MI355X: 10 %
-// rms (9 % on 11 310 of 900 others) where a FLOP rate missed by 22 %.
+// workgroups (the last round partly empty), `alone` for each K step of one workgroup and `more` for each step of the share
+// past the first; the repack, the output and the reduce at their traffic, common to all. Fitted to 37 828 timings of 3044
+// layers on one MI355X: 9 % rms, as much on 11 310 of 900 others, where a FLOP rate missed by 22 %.
 struct Cost {
   int tile_m, tile_n, tile_k, waves_m, waves_n;
   double fixed, odd_y, first, alone, more;
 };
 constexpr Cost kCosts[] = {
-    {64, 32, 64, 2, 1, 3.58, 0.89, 0.84, 0.331, 0.121},
-    {64, 64, 32, 2, 2, 3.32, 0.82, 1.03, 0.221, 0.112},
-    {64, 64, 64, 2, 2, 3.35, 0.88, 1.61, 0.361, 0.204},
-    {64, 64, 64, 4, 2, 3.33, 0.79, 1.72, 0.356, 0.198},
-    {64, 128, 32, 2, 2, 4.21, 1.74, 2.11, 0.336, 0.197},
-    {64, 128, 64, 2, 2, 3.91, 2.07, 4.54, 0.582, 0.560},
-    {64, 128, 64, 2, 4, 4.06, 1.35, 2.43, 0.461, 0.296},
-    {64, 128, 128, 2, 4, 3.70, 1.46, 3.91, 0.887, 0.823},
-    {64, 256, 64, 2, 4, 5.12, 2.53, 3.87, 0.736, 0.767},
-    {128, 64, 32, 2, 2, 3.85, 1.85, 1.91, 0.305, 0.170},
-    {128, 64, 64, 2, 2, 4.15, 1.91, 2.09, 0.559, 0.259},
-    {128, 64, 64, 4, 2, 3.58, 1.49, 2.18, 0.502, 0.265},
-    {128, 64, 128, 4, 2, 3.40, 1.60, 3.71, 0.811, 0.734},
-    {128, 128, 32, 2, 2, 5.89, 3.40, 2.49, 0.433, 0.251},
-    {128, 128, 32, 2, 4, 4.33, 2.51, 3.64, 0.410, 0.416},
-    {128, 128, 64, 2, 2, 6.02, 3.75, 5.15, 0.680, 1.010},
-    {128, 128, 64, 4, 2, 4.81, 2.71, 3.95, 0.624, 0.580},
-    {128, 128, 128, 4, 2, 5.05, 2.65, 4.71, 1.160, 1.362},
-    {128, 256, 32, 2, 4, 6.86, 3.83, 5.07, 0.506, 0.917},
-    {256, 128, 32, 4, 2, 6.41, 4.46, 5.03, 0.463, 0.900},
+    {64, 32, 64, 2, 1, 3.34, 0.74, 0.81, 0.322, 0.111},
+    {64, 64, 32, 2, 2, 3.04, 0.66, 0.89, 0.214, 0.103},
+    {64, 64, 64, 2, 2, 2.76, 0.69, 1.55, 0.355, 0.191},
+    {64, 64, 64, 4, 2, 2.73, 0.47, 1.68, 0.347, 0.185},
+    {64, 128, 32, 2, 2, 3.50, 1.45, 2.03, 0.325, 0.169},
+    {64, 128, 64, 2, 2, 2.03, 1.75, 4.79, 0.575, 0.496},
+    {64, 128, 64, 2, 4, 3.42, 0.99, 2.21, 0.429, 0.290},
+    {64, 128, 128, 2, 4, 2.20, 1.09, 3.95, 0.870, 0.785},
+    {64, 256, 64, 2, 4, 3.65, 2.33, 3.86, 0.695, 0.635},
+    {128, 64, 32, 2, 2, 3.28, 1.54, 1.80, 0.294, 0.150},
+    {128, 64, 64, 2, 2, 3.51, 1.62, 1.94, 0.538, 0.233},
+    {128, 64, 64, 4, 2, 3.02, 1.24, 1.95, 0.467, 0.264},
+    {128, 64, 128, 4, 2, 2.01, 1.29, 3.74, 0.793, 0.681},
+    {128, 128, 32, 2, 2, 4.96, 3.16, 2.38, 0.418, 0.215},
+    {128, 128, 32, 2, 4, 2.92, 2.25, 3.62, 0.397, 0.378},
+    {128, 128, 64, 2, 2, 3.62, 3.60, 5.95, 0.647, 0.769},
+    {128, 128, 64, 4, 2, 3.13, 2.47, 4.17, 0.601, 0.437},
+    {128, 128, 128, 4, 2, 2.95, 2.39, 5.03, 1.137, 1.129},
+    {128, 256, 32, 2, 4, 4.27, 3.65, 5.55, 0.504, 0.732},
+    {256, 128, 32, 4, 2, 4.19, 4.31, 5.26, 0.450, 0.810},
 };
 
 const Cost* cost_of(const gie_igemm_config& c) {
@@ -171,10 +171,11 @@ struct Fns {
     const double y = double(p.output_shape().numel()) * 2.0 / 1e6;
     const double odd_x = int64_t(p.in_h) * p.in_w % 4 != 0 ? 1.0 : 0.0, odd_y = int64_t(p.out_h()) * p.out_w() % 4 != 0 ? 1.0 : 0.0;
     const double steps = std::ceil(taps * cp / en.info.tile_k) / en.split;
-    const double share = double(blocks(prob)) / std::max(cus, 1);
-    const double reduce = en.split > 1 ? 0.33 * (en.split + 1) * 2.0 * y : 0.0;
-    return k.fixed + 1.58 * odd_x + k.odd_y * odd_y + (0.22 + 0.12 * odd_x) * moved + 0.51 * weights +
-           (0.08 + 0.35 * odd_y) * y + reduce + k.first * share + steps * (k.alone + std::max(0.0, share - 1.0) * k.more);
+    const double rounds = double(blocks(prob)) / std::max(cus, 1);
+    const double share = 0.5 * (rounds + std::ceil(rounds));  // the last round is partly empty
+    const double reduce = en.split > 1 ? 0.35 * (en.split + 1) * 2.0 * y : 0.0;
+    return k.fixed + 1.82 * odd_x + k.odd_y * odd_y + (0.23 + 0.11 * odd_x) * moved + 0.56 * weights +
+           (0.14 + 0.35 * odd_y) * y + reduce + k.first * share + steps * (k.alone + std::max(0.0, share - 1.0) * k.more);
   }
   static int occupancy(const ConvProblem& prob) {
     int n = 1;

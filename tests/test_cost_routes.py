@@ -42,10 +42,12 @@ def _us(p):
     (P(15, 352, 32, 32, 272, 3, 3, 1, 1, 1, 1, precision="bf16", has_bias=False, relu=False), "nhwc_bf16_128x256x64_sk1",
      "band_bf16_3x3_32x224x32_s4_sk1"),
     (P(6, 256, 33, 33, 64, 3, 3, 2, 2, 1, 1, precision="bf16"), "nhwc_bf16_64x64x64_sk4", "band_bf16_3x3_32x256x32_s3_sk4"),
-    # the implicit GEMM over images of no multiple of four pixels: 20.3 and 31.2 us, 47.2 and 78.3; its tiles: 31.2 and 26.2
+    # the implicit GEMM over images of no multiple of four pixels: 20.3 and 31.2 us, 47.2 and 78.3; its rounds: 46.8 and
+    # 68.0, 22.5 and 28.6
     (P(4, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x64x32_w2x2_s4_sk1"),
     (P(14, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x128x32_w2x2_s4_sk1"),
-    (P(4, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "mfma_fp16_128x128x32_w2x2_s4_sk1", "mfma_fp16_64x64x32_w2x2_s4_sk1"),
+    (P(2, 464, 46, 46, 464, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_128x128x64_sk1", "mfma_bf16_128x64x128_w4x2_s2_sk1"),
+    (P(11, 130, 44, 15, 288, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_128x128x64_sk1", "mfma_bf16_64x128x64_w2x4_s4_sk1"),
     # small convolutions in whole rounds of workgroups: 7.1 and 10.1 us, 12.9 and 19.7, 6.4 and 9.6
     (P(16, 32, 12, 12, 128, 1, 3, 1, 1, 0, 1, precision="bf16", relu=False), "nhwc_bf16_64x64x64_sk1", "mini_bf16_32x32_k8w"),
     (P(26, 416, 33, 33, 32, 1, 1, precision="fp16"), "gather_fp16_1x1_64x128_t256", "mini_fp16_32x32_k8w"),

@@ -92,7 +92,10 @@ double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   const double share = std::max(1.0, double(blocks_of(config, prob)) / std::max(cus, 1));
   const double rounds = f.overlap * share + (1.0 - f.overlap) * std::ceil(share);
   const double spread = p.stride_w > 1 ? 1.0 + f.strided : 1.0, ragged = k16 && p.gemm_k() % 2 != 0 ? 1.0 + f.ragged : 1.0;
-  return rounds * (f.start + loads * f.load * spread * ragged + double((steps + nw - 1) / nw) * f.step);
+  // sixteen waves on the same supersteps: 3x3 1 % faster (their stores spread over more threads), 1 % slower where they set
+  // up a table of taps
+  const double wide = nw != 16 || one ? 0.0 : nine ? -0.04 : 0.08;
+  return rounds * (f.start + wide + loads * f.load * spread * ragged + double((steps + nw - 1) / nw) * f.step);
 }
 
 int mini_best_config(const ConvProblem& prob, int cus, double* us) {

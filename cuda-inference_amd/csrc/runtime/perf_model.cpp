@@ -7,9 +7,11 @@
 //   fixed   = launches x dispatch cost + the family's cost of filling and draining a launch
 //   serial  = passes that do not overlap the main kernel (KernelDesc::serial_us: a repack, a reduce)
 //   time    = max(compute, memory) + fixed + serial  (reported as launch_us; "launch"-bound when it dominates)
-// A family with a formula of its own (KernelDesc::busy_us: everything but dispatch) is timed as max(busy, memory) +
-// dispatch; compute, memory and fixed stay the roofline's parts, by which the estimate is called compute-, bandwidth- or
-// launch-bound.
+// A family with a formula of its own (KernelDesc::busy_us: everything but dispatch, its traffic too) is timed as busy +
+// dispatch, and not below its traffic at the HBM's full rate; compute, memory and fixed stay the roofline's parts, by which
+// the estimate is called compute-, bandwidth- or launch-bound. (The family's HBM efficiency is no bound for it: tensors that
+// the Infinity Cache holds between calls move faster, 1x1 256 -> 128 over 56x56, batch 32, at 4.0 TB/s on the streaming
+// pointwise kernel.)
 // * Family efficiencies are not guesses per backend: each is what that kernel family reached on an MI355X in the
 //   library's benchmark protocol (per-call time, inputs resident in HBM), listed in kFamilies with the measurement.
 // * Wave efficiency follows how gfx950 places workgroups: dispatch deals them round-robin to the 8 XCDs, and each
@@ -63,8 +65,7 @@ constexpr FamilyProfile kFamilies[] = {
     {"halo_", 0.37, 0.40, 10.0},    // L2 23.3 us including the repack launch, L5 24.7 us at split 4
     {"mfma_", 0.22, 0.35, 8.0},     // L2 25.7 us, L3 87 us, L4 145 us, L5 26.0 us at split 4
     {"pw_", 0.30, 0.48, 2.0},       // L3 37.2-39.6 us (weight-stationary streaming form; shared tiles, 128-byte
-                                    // device-scope runs) = 3.3-3.5 TB/s of compulsory traffic (the bound its entries'
-                                    // own formulas are held to)
+                                    // device-scope runs) = 3.3-3.5 TB/s of compulsory traffic
     {"stem_", 0.28, 0.69, 2.0},     // L4 26.6-26.8 us (128-byte device-scope output runs) = 4.6 TB/s
     {"narrow_", 0.084, 0.30, 2.0},  // L5 15.0 us (123 TFLOP/s)
     {"stack_", 0.33, 0.40, 4.1},    // L5 9.6 us at split 2 (6.7 conv + 2.8 reduce), 10.2 at split 1
@@ -325,7 +326,7 @@ Estimate estimate_kernel(const ConvProblem& prob, const KernelDesc& k, const Dev
     }
   }
   e.bound = bound_of(e.compute_us, e.memory_us, e.launch_us);
-  e.time_us = std::max(busy_us, e.memory_us) + (k.busy_us ? dispatch_us : e.launch_us) +
+  e.time_us = std::max(busy_us, k.busy_us ? e.memory_us * hbm_eff : e.memory_us) + (k.busy_us ? dispatch_us : e.launch_us) +
               (k.serial_us ? k.serial_us(prob) : 0.0);
   return e;
 }

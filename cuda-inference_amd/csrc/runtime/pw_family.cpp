@@ -105,12 +105,12 @@ struct Fns {
   // Tiled: fixed cost, then one workgroup's 32-channel steps or a CU's share of the workgroups at a start-up and a cost
   // for each step; its BF16 form rounds with integer arithmetic, which shows as 1.65 us a launch. Streaming: the weights
   // (by the k-steps that their registers hold) once for each round of workgroups an XCD's 32 CUs take, then a CU's
-  // 64-pixel blocks. Both store at a cost for each MB of y. Where x and y pass 80 MB they no longer stay in the Infinity
-  // Cache between calls on a few sets of tensors, and a MB beyond costs more, most where image rows of y share 128-byte
-  // lines. Fitted to 1316 and 787 layers on one MI355X (7 to 56 a side, 16 to 1024 channels, three sets in turn): 6 % and
-  // 8 % rms, 5 % and 7 % on 82 and 57 others. A FLOP rate put the tiled form first where the streaming one is faster
-  // (256 -> 1024 over 28x28, batch 64: 83.9 and 53.7 us) and the gathering kernel before the tiled form (512 -> 128 over
-  // 28x28, batch 32: 13.2 and 10.3 us).
+  // 64-pixel blocks. Both store at a cost for each MB of y, and the streaming form reads at the same for x. Where x and y
+  // pass 80 MB they no longer stay in the Infinity Cache between calls on a few sets of tensors, and a MB beyond costs more,
+  // most where image rows of y share 128-byte lines. Fitted to 1316 and 787 layers on one MI355X (7 to 56 a side, 16 to 1024
+  // channels, three sets in turn): 6 % and 7 % rms, 5 % and 6 % on 82 and 57 others. A FLOP rate put the tiled form first
+  // where the streaming one is faster (256 -> 1024 over 28x28, batch 64: 83.9 and 53.7 us) and the gathering kernel before
+  // the tiled form (512 -> 128 over 28x28, batch 32: 13.2 and 10.3 us).
   static double busy_us(const ConvProblem& prob, int cus) {
     const Conv2DParams& p = prob.p;
     cus = std::max(cus, 1);
@@ -131,10 +131,10 @@ struct Fns {
     const int64_t ranges = std::max<int64_t>(1, std::min<int64_t>(n_blk, std::max<int64_t>(1, cus / n_ob)));
     const int64_t per_xcd = std::max(cus / 8, 1);
     const double rounds = double(((ranges + 7) / 8 * n_ob + per_xcd - 1) / per_xcd);
-    const double blocks_each = double((n_blk + ranges - 1) / ranges);
+    const double blocks_each = 0.5 * (double((n_blk + ranges - 1) / ranges) + double(n_blk) / double(ranges));
     const double ks = p.in_channels <= 64 ? 4.0 : p.in_channels <= 128 ? 8.0 : 16.0;
-    return 1.45 + rounds * (0.137 * ks + blocks_each * (0.5 + 0.055 * ks)) + 0.111 * y +
-           (shared_lines ? 0.37 : 0.17) * spilled;
+    return 1.4 + rounds * (0.137 * ks + blocks_each * (0.56 + 0.054 * ks)) + 0.085 * (x + y) +
+           (shared_lines ? 0.40 : 0.15) * spilled;
   }
   static void launch(const LaunchArgs& la) {
     const ConvProblem& prob = *la.problem;

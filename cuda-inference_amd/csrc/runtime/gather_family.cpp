@@ -82,33 +82,36 @@ struct Fns {
   // workgroup's latency (`alone`) plus, beyond 0.75 workgroups a CU, its share of them (`step`); both grow with the step's
   // vector loads (16 clocks each: a wave's x loads cover 64 pixel groups, its w loads 8 rows) and where channels end
   // inside a step (`part`); then the output stores, and more for each MB of x and y past the 80 that stay in the
-  // Infinity Cache over a few sets of tensors (`spill`, `spill_lines` where image rows of y share 128-byte lines). Fitted
-  // per tile to 2106-2199 layers on one MI355X (7 to 56 a side, 16 to 1992 channels, both strides): 8-11 % rms, 8-12 % on
-  // 323-335 others.
+  // Infinity Cache over a few sets of tensors (`spill`, `spill_lines` where image rows of y share 128-byte lines). A strided
+  // row of x takes twice the cache lines: dearer loads alone and shared (`lines`), and each filter tile reads the rows'
+  // lines again (`again`, per MB: 1920 -> 1920 over 33x33, batch 7, 58 us; without it 38). Fitted per tile to 2366-2699
+  // layers on one MI355X (7 to 56 a side, 16 to 2000 channels, both strides): 8-11 % rms, 8-11 % on 523-535 others.
   static double busy_us(const ConvProblem& prob, int cus) {
     struct Fit {
-      double fixed, alone, alone_load, step, step_load, out, odd, part, spill, spill_lines;
+      double fixed, alone, alone_load, step, step_load, out, odd, part, spill, spill_lines, lines, lines_shared, again;
     };
-    constexpr Fit kFit[] = {{2.07, 0.286, 0.818, 0.148, 0.300, 0.329, 0.89, 0.57, 0.35, 0.28},
-                            {2.24, 0.390, 0.619, 0.290, 0.384, 0.224, 1.04, 0.19, 0.28, 0.19},
-                            {3.07, 0.538, 0.643, 0.456, 0.450, 0.235, 1.52, 0.15, 0.26, 0.14},
-                            {3.16, 0.480, 0.740, 0.169, 1.742, 0.261, 1.37, 0.20, 0.14, 0.16}};
+    constexpr Fit kFit[] = {{2.10, 0.291, 0.776, 0.155, 0.267, 0.331, 0.96, 0.55, 0.34, 0.28, 0.15, 0.00, 0.077},
+                            {2.25, 0.416, 0.529, 0.294, 0.379, 0.225, 1.14, 0.18, 0.25, 0.20, 0.61, 0.37, 0.068},
+                            {3.09, 0.568, 0.553, 0.461, 0.433, 0.238, 1.66, 0.14, 0.26, 0.13, 0.67, 1.51, 0.038},
+                            {3.13, 0.579, 0.613, 0.196, 1.667, 0.268, 1.52, 0.16, 0.14, 0.16, 0.72, 0.68, 0.048}};
     const Fit& f = kFit[Config];
     const Conv2DParams& p = prob.p;
     const Tile t = tile_of(Config);
-    const int64_t hw = int64_t(p.in_h) * p.in_w;
+    const int64_t hw = int64_t(p.in_h) * p.in_w, ohw = int64_t(p.out_h()) * p.out_w();
     const bool flat = p.stride_h == 1 && p.stride_w == 1 && p.pad_h == 0 && p.pad_w == 0;
     const int px = std::min(flat && hw % 4 == 0 ? 4 : flat && hw % 2 == 0 ? 2 : 1, t.m == 256 ? 2 : 4);
-    // a strided row of x takes twice the cache lines (256 -> 512, 56x56 /2, batch 32: 38 us at 128x128)
-    const double spread = p.stride_w > 1 ? 1.35 : 1.0;
-    const double loads = (spread * double(t.n) / px + t.m / 8.0) * 16.0 / 2400.0;  // us of a step's vector loads
+    const double strided = p.stride_w > 1 ? 1.0 : 0.0;
+    const double x_loads = double(t.n) / px * 16.0 / 2400.0, w_loads = t.m / 8.0 * 16.0 / 2400.0;  // us of a step's loads
     const double steps = double((p.in_channels + 63) / 64), share = double(blocks(prob)) / std::max(cus, 1);
-    const double y = double(p.output_shape().numel()) * 2.0 / 1e6, x = double(p.input_shape().numel()) * 2.0 / 1e6;
-    const int64_t ohw = int64_t(p.out_h()) * p.out_w();
+    const double y = double(p.output_shape().numel()) * 2.0 / 1e6;
+    const double x = double(p.input_shape().numel()) * 2.0 / 1e6 / p.stride_h;  // MB of the rows that are read
     const double spill = std::max(0.0, x + y - 80.0) * (f.spill + (ohw % 64 != 0 ? f.spill_lines : 0.0));
-    const double step = f.alone + f.alone_load * loads + std::max(0.0, share - 0.75) * (f.step + f.step_load * loads);
+    const double step = f.alone + f.alone_load * (x_loads * (1.0 + f.lines * strided) + w_loads) +
+                        std::max(0.0, share - 0.75) *
+                            (f.step + f.step_load * (x_loads * (1.0 + f.lines_shared * strided) + w_loads));
     const double part = p.in_channels % 64 != 0 ? 1.0 + f.part : 1.0;
-    return f.fixed + (ohw % 8 != 0 ? f.odd : 0.0) + steps * step * part + f.out * y + spill;
+    const double again = strided * f.again * x * double((p.out_channels + t.m - 1) / t.m);
+    return f.fixed + (ohw % 8 != 0 ? f.odd : 0.0) + steps * step * part + f.out * y + again + spill;
   }
   static void launch(const LaunchArgs& la) {
     if (la.only_stage >= 0 && la.only_stage != 1) return;  // one stage: the convolution itself

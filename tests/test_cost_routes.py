@@ -48,6 +48,9 @@ def _us(p):
     (P(14, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x128x32_w2x2_s4_sk1"),
     (P(2, 464, 46, 46, 464, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_128x128x64_sk1", "mfma_bf16_128x64x128_w4x2_s2_sk1"),
     (P(11, 130, 44, 15, 288, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_128x128x64_sk1", "mfma_bf16_64x128x64_w2x4_s4_sk1"),
+    # strided rows that every filter tile reads again: 18.7 and 31.9 us, 35.2 and 56.2
+    (P(4, 1408, 24, 24, 1408, 1, 1, 2, 2, precision="bf16"), "mfma_bf16_64x64x64_w4x2_s4_sk1", "gather_bf16_1x1_64x64_t128"),
+    (P(4, 1920, 34, 34, 1920, 1, 1, 2, 2, precision="fp16"), "nhwc_fp16_128x128x64_sk1", "gather_fp16_1x1_64x64_t128"),
     # small convolutions in whole rounds of workgroups: 7.1 and 10.1 us, 12.9 and 19.7, 6.4 and 9.6
     (P(16, 32, 12, 12, 128, 1, 3, 1, 1, 0, 1, precision="bf16", relu=False), "nhwc_bf16_64x64x64_sk1", "mini_bf16_32x32_k8w"),
     (P(26, 416, 33, 33, 32, 1, 1, precision="fp16"), "gather_fp16_1x1_64x128_t256", "mini_fp16_32x32_k8w"),

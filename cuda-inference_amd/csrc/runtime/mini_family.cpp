@@ -67,20 +67,21 @@ int64_t blocks_of(int config, const ConvProblem& prob) {
 // One workgroup runs on a CU at a time, so a launch takes whole rounds of them: 1x3 32 -> 32 over 32x32, BF16, takes
 // 5.7 us at 128 to 256 workgroups, 10.0 to 10.2 at 288 to 512, 14.5 at 544 to 640. A round costs `start` (pixel set-up,
 // partial tiles, stores), each operand load of a lane `load` and each superstep of the longest wave's share `step`; with
-// 16x16 tiles over few channels the rounds overlap in part. Strided rows of x take more cache lines (`strided`), odd
-// 16-bit rows of weights element loads (`ragged`). Fitted per type, filter and tile to 95-3907 timings on one MI355X: 5-13 %
-// rms, 5-13 % on 19-720 others.
+// 16x16 tiles over few channels the rounds overlap in part. Strided rows of x take more cache lines (`strided`), which
+// every filter tile of a 1x1 layer reads `again`; odd 16-bit rows of weights take element loads (`ragged`). 1x1 layers, up
+// to 2000 channels of tens of images, are priced for their MB of x and y too. Fitted per type, filter and tile to 95-4835
+// timings on one MI355X: 5-13 % rms, 5-13 % on 19-1024 others.
 double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   struct Fit {
-    double start, load, step, overlap, strided, ragged;
+    double start, load, step, overlap, strided, ragged, again, x, y;
   };
   constexpr Fit kFit[2][3][2] = {  // 16 / 32 bits; 1x1, 3x3, other filters; 16x16, 32x32 tiles
-      {{{1.43, 0.0062, 0.107, 0.47, 0.49, 1.60}, {1.44, 0.0055, 0.332, 0.00, 0.56, 1.77}},
-       {{1.44, 0.0079, 0.082, 0.11, 0.21, 1.37}, {1.48, 0.0073, 0.068, 0.04, 0.31, 1.51}},
-       {{1.63, 0.0061, 0.854, 0.00, 0.00, 1.90}, {2.23, 0.0059, 1.431, 0.00, 0.00, 1.30}}},
-      {{{1.12, 0.0071, 0.579, 0.35, 0.50, 0.00}, {1.39, 0.0102, 0.677, 0.00, 0.40, 0.00}},
-       {{1.81, 0.0096, 0.616, 0.08, 0.24, 0.00}, {2.10, 0.0098, 0.867, 0.09, 0.24, 0.00}},
-       {{1.86, 0.0113, 0.280, 0.00, 0.73, 0.00}, {2.60, 0.0136, 0.455, 0.00, 0.46, 0.00}}}};
+      {{{1.33, 0.0052, 0.191, 0.47, 0.00, 2.04, 0.043, 0.325, 0.00}, {1.34, 0.0052, 0.298, 0.00, 0.23, 1.80, 0.042, 0.139, 0.30}},
+       {{1.44, 0.0079, 0.082, 0.11, 0.21, 1.37, 0.0, 0.0, 0.0}, {1.48, 0.0073, 0.068, 0.04, 0.31, 1.51, 0.0, 0.0, 0.0}},
+       {{1.63, 0.0061, 0.854, 0.00, 0.00, 1.90, 0.0, 0.0, 0.0}, {2.23, 0.0059, 1.431, 0.00, 0.00, 1.30, 0.0, 0.0, 0.0}}},
+      {{{1.24, 0.0058, 0.445, 0.45, 0.07, 0.00, 0.012, 0.255, 0.00}, {1.14, 0.0088, 0.747, 0.11, 0.12, 0.00, 0.042, 0.076, 0.40}},
+       {{1.81, 0.0096, 0.616, 0.08, 0.24, 0.00, 0.0, 0.0, 0.0}, {2.10, 0.0098, 0.867, 0.09, 0.24, 0.00, 0.0, 0.0, 0.0}},
+       {{1.86, 0.0113, 0.280, 0.00, 0.73, 0.00, 0.0, 0.0, 0.0}, {2.60, 0.0136, 0.455, 0.00, 0.46, 0.00, 0.0, 0.0, 0.0}}}};
   const Conv2DParams& p = prob.p;
   const bool k16 = half_precision(prob.precision), one = p.kernel_h * p.kernel_w == 1;
   const bool nine = p.kernel_h == 3 && p.kernel_w == 3;
@@ -95,7 +96,11 @@ double mini_busy_us(int config, const ConvProblem& prob, int cus) {
   // sixteen waves on the same supersteps: 3x3 1 % faster (their stores spread over more threads), 1 % slower where they set
   // up a table of taps
   const double wide = nw != 16 || one ? 0.0 : nine ? -0.04 : 0.08;
-  return rounds * (f.start + wide + loads * f.load * spread * ragged + double((steps + nw - 1) / nw) * f.step);
+  const double es = k16 ? 2.0 : 4.0, y = double(p.output_shape().numel()) * es / 1e6;
+  const double x = double(p.input_shape().numel()) * es / 1e6 / (one ? p.stride_h : 1);  // MB of the rows that are read
+  const double again = p.stride_w > 1 ? f.again * x * double((p.out_channels + t - 1) / t) : 0.0;
+  return rounds * (f.start + wide + loads * f.load * spread * ragged + double((steps + nw - 1) / nw) * f.step) + f.x * x +
+         f.y * y + again;
 }
 
 int mini_best_config(const ConvProblem& prob, int cus, double* us) {

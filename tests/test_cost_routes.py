@@ -48,6 +48,9 @@ def _us(p):
     (P(14, 3, 225, 225, 96, 7, 7, 2, 2, 3, 3, precision="fp16"), "nhwc_fp16_128x256x64_sk1", "mfma_fp16_64x128x32_w2x2_s4_sk1"),
     (P(2, 464, 46, 46, 464, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_128x128x64_sk1", "mfma_bf16_128x64x128_w4x2_s2_sk1"),
     (P(11, 130, 44, 15, 288, 3, 3, 1, 1, 1, 1, precision="bf16"), "nhwc_bf16_128x128x64_sk1", "mfma_bf16_64x128x64_w2x4_s4_sk1"),
+    # large strided 1x1 layers are no small convolutions: 18.1 and 27.4 us, 26.5 and 40.2
+    (P(59, 744, 23, 23, 33, 1, 1, 2, 2, precision="bf16"), "gather_bf16_1x1_64x64_t128", "mini_bf16_32x32_k16w"),
+    (P(42, 836, 14, 30, 224, 1, 1, 2, 2, precision="fp16"), "gather_fp16_1x1_64x64_t128", "mini_fp16_32x32_k16w"),
     # strided rows that every filter tile reads again: 18.7 and 31.9 us, 35.2 and 56.2
     (P(4, 1408, 24, 24, 1408, 1, 1, 2, 2, precision="bf16"), "mfma_bf16_64x64x64_w4x2_s4_sk1", "gather_bf16_1x1_64x64_t128"),
     (P(4, 1920, 34, 34, 1920, 1, 1, 2, 2, precision="fp16"), "nhwc_fp16_128x128x64_sk1", "gather_fp16_1x1_64x64_t128"),
